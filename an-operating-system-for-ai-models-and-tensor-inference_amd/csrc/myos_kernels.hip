@@ -858,7 +858,8 @@ __global__ void rope_apply_kernel(float *x, size_t len, size_t head_dim, const f
   x[i1] = x1 * c.x + x0 * c.y;
 }
 
-// Op-tier gqa_attn_f32 for any shape: one workgroup per query head; scores
+// Op-tier gqa_attn_f32 for the shapes gqa_chunk_kernel does not take (any head
+// dim, any alignment): one workgroup per query head; scores
 // in a global scratch row of length seq; the last head's probabilities are
 // also written to `probs` (gqa.rs:26-30).
 __global__ void __launch_bounds__(kBlock)
@@ -906,6 +907,189 @@ __global__ void __launch_bounds__(kBlock)
       if (kept(t)) acc = fmaf(s[t], v[((size_t)g * seq + t) * d + j], acc);
     y[(size_t)h * d + j] = acc;
   }
+}
+
+// gqa_attn_f32 for head dims up to 256 that are multiples of 4 (16-byte aligned
+// operands): workgroup (c, h) takes positions [c * cp, (c + 1) * cp) of query
+// head h. K rows go to 16-lane groups (a lane holds columns 4 l + 64 i), four
+// positions per group in flight; the chunk's softmax is taken against its own
+// maximum, and V rows are summed by column groups over 512 / CG position
+// streams. With one chunk the result is final; otherwise the chunk leaves
+// (o[d], max, sum) in part and gqa_merge_kernel combines them. K and V are read
+// in 16-byte lane loads by every CU the chunks fill, where the one-workgroup-
+// per-head kernel walks each K row in a single lane: 12 q / 2 kv heads of 128,
+// 2304 positions, 776 -> 31 us per call (most of it then host work).
+constexpr int kGqaThreads = 512, kGqaMaxChunk = 1024;
+
+template <int NJ>
+__global__ void __launch_bounds__(kGqaThreads)
+    gqa_chunk_kernel(float *y, const float *q, const float *k, const float *v, float *probs, float *scr,
+                     float *part, int nq, int nkv, int d, int seq, int seen, int cp) {
+  constexpr int CG = 16 * NJ;             // 4-column groups, d / 4 of them in use
+  constexpr int NS = kGqaThreads / CG;    // position streams of the V sum
+  constexpr int U = 4, UV = 4;
+  __shared__ float sc[kGqaMaxChunk];
+  __shared__ float red[kGqaThreads / kWave];
+  __shared__ float4 osum[kGqaThreads];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int nc = gridDim.x, c = blockIdx.x, h = blockIdx.y, g = h / (nq / nkv);
+  const int t0 = c * cp, n = min(cp, seen - t0);
+  const float scale = 1.0f / sqrtf((float)d);
+  const float *kb = k + ((size_t)g * seq + t0) * d, *vb = v + ((size_t)g * seq + t0) * d;
+  const int l16 = tid & 15;
+  float4 qv[NJ];
+#pragma unroll
+  for (int i = 0; i < NJ; i++) {
+    const int j = 4 * l16 + 64 * i;
+    qv[i] = j < d ? *(const float4 *)(q + (size_t)h * d + j) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  constexpr int PG = kGqaThreads / 16;  // positions per round of one position per group
+  for (int r0 = tid >> 4; r0 < n; r0 += PG * U) {
+    float4 kv[U][NJ];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int i = 0; i < NJ; i++) {
+        const int r = min(r0 + u * PG, n - 1), j = 4 * l16 + 64 * i;  // clamped, unconditional
+        kv[u][i] = *(const float4 *)(kb + (size_t)r * d + (j < d ? j : 0));
+      }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      float acc = 0.f;
+#pragma unroll
+      for (int i = 0; i < NJ; i++)
+        if (4 * l16 + 64 * i < d) {
+          acc = fmaf(qv[i].x, kv[u][i].x, acc);
+          acc = fmaf(qv[i].y, kv[u][i].y, acc);
+          acc = fmaf(qv[i].z, kv[u][i].z, acc);
+          acc = fmaf(qv[i].w, kv[u][i].w, acc);
+        }
+      acc = group_sum<16>(acc) * scale;
+      const int r = r0 + u * PG;
+      if (l16 == 0 && r < n) sc[r] = acc;
+    }
+  }
+  __syncthreads();
+  auto block_red = [&](float x, bool mx) {
+    x = mx ? group_max<kWave>(x) : group_sum<kWave>(x);
+    __syncthreads();
+    if (lane == 0) red[wave] = x;
+    __syncthreads();
+    float t = red[0];
+#pragma unroll
+    for (int w = 1; w < kGqaThreads / kWave; w++) t = mx ? fmaxf(t, red[w]) : t + red[w];
+    return t;
+  };
+  float mx = -INFINITY;
+  for (int t = tid; t < n; t += kGqaThreads) mx = fmaxf(mx, sc[t]);  // NaN scores never win
+  mx = block_red(mx, true);
+  // a chunk whose scores are all -inf weighs nothing next to finite ones; as the
+  // only chunk its exponentials are NaN, as the whole row's are
+  const float ref = nc > 1 && mx == -INFINITY ? 0.f : mx;
+  float sum = 0.f;
+  for (int t = tid; t < n; t += kGqaThreads) {
+    const float s = sc[t], e = expf(s - ref);
+    if (nc > 1) scr[(size_t)h * seq + t0 + t] = s;
+    sc[t] = e;
+    sum += e;
+  }
+  sum = block_red(sum, false);
+  if (nc == 1) {
+    for (int t = tid; t < n; t += kGqaThreads) sc[t] = sc[t] / sum;
+    __syncthreads();
+    if (h == nq - 1)
+      for (int t = tid; t < seq; t += kGqaThreads) probs[t] = t < n ? sc[t] : 0.f;
+  }
+  const int cg = tid % CG, st = tid / CG, j = 4 * cg;
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (j < d) {
+    int t = st;
+    for (; t + (UV - 1) * NS < n; t += UV * NS) {
+      float4 vv[UV];
+#pragma unroll
+      for (int u = 0; u < UV; u++) vv[u] = *(const float4 *)(vb + (size_t)(t + u * NS) * d + j);
+#pragma unroll
+      for (int u = 0; u < UV; u++) {
+        const float p = sc[t + u * NS];
+        o.x = fmaf(p, vv[u].x, o.x);
+        o.y = fmaf(p, vv[u].y, o.y);
+        o.z = fmaf(p, vv[u].z, o.z);
+        o.w = fmaf(p, vv[u].w, o.w);
+      }
+    }
+    for (; t < n; t += NS) {
+      const float4 vv = *(const float4 *)(vb + (size_t)t * d + j);
+      const float p = sc[t];
+      o.x = fmaf(p, vv.x, o.x);
+      o.y = fmaf(p, vv.y, o.y);
+      o.z = fmaf(p, vv.z, o.z);
+      o.w = fmaf(p, vv.w, o.w);
+    }
+  }
+  osum[tid] = o;
+  __syncthreads();
+  if (tid < CG && j < d) {
+    for (int s2 = 1; s2 < NS; s2++) {
+      const float4 w = osum[s2 * CG + tid];
+      o.x += w.x;
+      o.y += w.y;
+      o.z += w.z;
+      o.w += w.w;
+    }
+    float *dst = nc == 1 ? y + (size_t)h * d : part + ((size_t)h * nc + c) * (d + 4);
+    *(float4 *)(dst + j) = o;
+    if (nc > 1 && tid == 0) {
+      dst[d] = mx;
+      dst[d + 1] = sum;
+    }
+  }
+}
+
+// The chunks of head blockIdx.x in chunk order, and the last head's
+// probabilities. An output that is not finite is recomputed from the scores as
+// the row-wide softmax times V, position by position: there a probability that
+// is zero next to the row's maximum (but not next to its chunk's) meets an
+// infinite value as 0 x inf.
+__global__ void __launch_bounds__(kBlock)
+    gqa_merge_kernel(float *y, const float *v, float *probs, const float *scr, const float *part, int nq,
+                     int nkv, int d, int seq, int seen, int nc) {
+  __shared__ float red4[4];
+  const int h = blockIdx.x, tid = threadIdx.x, pd = d + 4;
+  const float *ph = part + (size_t)h * nc * pd;
+  const float *s = scr + (size_t)h * seq;
+  float mx = -INFINITY;
+  for (int c = tid; c < nc; c += kBlock) mx = fmaxf(mx, ph[(size_t)c * pd + d]);
+  mx = group_max<kWave>(mx);
+  if ((tid & 63) == 0) red4[tid >> 6] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(red4[0], red4[1]), fmaxf(red4[2], red4[3]));
+  float sum = 0.f;
+  for (int c = tid; c < nc; c += kBlock) sum += ph[(size_t)c * pd + d + 1] * expf(ph[(size_t)c * pd + d] - mx);
+  sum = block_sum(sum, red4);
+  for (int j = tid; j < d; j += kBlock) {
+    float acc = 0.f;
+    for (int c0 = 0; c0 < nc; c0 += 8) {
+      float o[8], m[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) {
+        const float *pc = ph + (size_t)min(c0 + u, nc - 1) * pd;
+        o[u] = pc[j];
+        m[u] = pc[d];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (c0 + u < nc) acc = fmaf(o[u], expf(m[u] - mx), acc);
+    }
+    acc /= sum;
+    if (!__builtin_isfinite(acc)) {
+      const float *vj = v + (size_t)(h / (nq / nkv)) * seq * d + j;
+      acc = 0.f;
+      for (int t = 0; t < seen; t++) acc = fmaf(expf(s[t] - mx) / sum, vj[(size_t)t * d], acc);
+    }
+    y[(size_t)h * d + j] = acc;
+  }
+  if (h == nq - 1)
+    for (int t = tid; t < seq; t += kBlock) probs[t] = t < seen ? expf(s[t] - mx) / sum : 0.f;
 }
 
 __global__ void swiglu_mul_kernel(float *h, const float *g, const float *u, size_t n) {
@@ -2924,11 +3108,56 @@ hipError_t launch_rope_apply(float *x, size_t len, size_t head_dim, const float2
   return hipGetLastError();
 }
 
+// Positions per chunk of gqa_chunk_kernel: about two chunks per CU over all
+// heads, 32 to kGqaMaxChunk positions. Up to 128 positions one chunk per head
+// (no merge launch) is ahead.
+static int gqa_chunk(int nq, int seen) {
+  if (seen <= 128) return 128;
+  const long per = (512 + nq - 1) / nq;  // chunks per head
+  const long cp = (((seen + per - 1) / per) + 31) & ~31L;
+  return (int)std::min<long>(std::max<long>(cp, 32), kGqaMaxChunk);
+}
+
+static bool gqa_chunked(const float *y, const float *q, const float *k, const float *v, int nq, int d) {
+  return (d & 3) == 0 && d <= 256 && nq <= 65535 &&
+         (((uintptr_t)y | (uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
+}
+
+static size_t gqa_align4(size_t n) { return (n + 3) & ~(size_t)3; }  // floats: keeps part 16-byte aligned
+
+size_t gqa_scratch_floats(const float *y, const float *q, const float *k, const float *v, int nq, int d,
+                          int seq, int mask, size_t query_pos) {
+  if (!gqa_chunked(y, q, k, v, nq, d)) return (size_t)nq * seq;
+  const int seen = mask && query_pos < (size_t)seq ? (int)query_pos + 1 : seq;
+  const int cp = gqa_chunk(nq, seen), nc = (int)(((long)seen + cp - 1) / cp);
+  return nc == 1 ? 0 : gqa_align4((size_t)nq * seq) + (size_t)nq * nc * (d + 4);
+}
+
 hipError_t launch_gqa_general(float *y, const float *q, const float *k, const float *v,
                               float *probs, float *scratch, int nq, int nkv, int d, int seq,
                               int mask, size_t query_pos, hipStream_t s) {
-  hipLaunchKernelGGL(gqa_general_kernel, dim3(nq), dim3(kBlock), 0, s, y, q, k, v, probs,
-                     scratch, nq, nkv, d, seq, mask, (unsigned long long)query_pos);
+  if (!gqa_chunked(y, q, k, v, nq, d)) {
+    hipLaunchKernelGGL(gqa_general_kernel, dim3(nq), dim3(kBlock), 0, s, y, q, k, v, probs,
+                       scratch, nq, nkv, d, seq, mask, (unsigned long long)query_pos);
+    return hipGetLastError();
+  }
+  const int seen = mask && query_pos < (size_t)seq ? (int)query_pos + 1 : seq;
+  const int cp = gqa_chunk(nq, seen), nc = (int)(((long)seen + cp - 1) / cp);
+  float *part = scratch + (nc == 1 ? 0 : gqa_align4((size_t)nq * seq));
+  const dim3 grid(nc, nq);
+  if (d <= 64)
+    hipLaunchKernelGGL(gqa_chunk_kernel<1>, grid, dim3(kGqaThreads), 0, s, y, q, k, v, probs, scratch, part,
+                       nq, nkv, d, seq, seen, cp);
+  else if (d <= 128)
+    hipLaunchKernelGGL(gqa_chunk_kernel<2>, grid, dim3(kGqaThreads), 0, s, y, q, k, v, probs, scratch, part,
+                       nq, nkv, d, seq, seen, cp);
+  else
+    hipLaunchKernelGGL(gqa_chunk_kernel<4>, grid, dim3(kGqaThreads), 0, s, y, q, k, v, probs, scratch, part,
+                       nq, nkv, d, seq, seen, cp);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || nc == 1) return e;
+  hipLaunchKernelGGL(gqa_merge_kernel, dim3(nq), dim3(kBlock), 0, s, y, v, probs, scratch, part, nq, nkv, d,
+                     seq, seen, nc);
   return hipGetLastError();
 }
 

@@ -198,12 +198,13 @@ int myos_gqa_attn_f32(float *y, size_t y_len, const float *q, size_t q_len, cons
   hipStream_t s = S(stream);
   size_t scr_elems;
   if (!mul_ok(num_q_heads, seq_len, &scr_elems)) return MYOS_E_SHAPE;
+  scr_elems = gqa_scratch_floats(y, q, k, v, (int)num_q_heads, (int)head_dim, (int)seq_len, mask, query_pos);
   float *scr = nullptr;
-  if (hipMallocAsync((void **)&scr, scr_elems * sizeof(float), s) != hipSuccess)
+  if (scr_elems && hipMallocAsync((void **)&scr, scr_elems * sizeof(float), s) != hipSuccess)
     return MYOS_E_HIP;
   hipError_t e = launch_gqa_general(y, q, k, v, probs, scr, (int)num_q_heads, (int)num_kv_heads,
                                     (int)head_dim, (int)seq_len, mask, query_pos, s);
-  hipError_t f = hipFreeAsync(scr, s);
+  hipError_t f = scr ? hipFreeAsync(scr, s) : hipSuccess;
   return hip_status(e != hipSuccess ? e : f);
 }
 

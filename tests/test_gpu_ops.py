@@ -276,3 +276,74 @@ def test_greedy_token(case):
         lg = np.full(5, -np.inf, np.float32)
         lg[3] = np.nan
     assert myos.greedy_token(dev(lg)) == oracle.greedy_token(lg)
+
+
+def _gqa64(q, k, v, n):
+    """Row-wide softmax attention in float64 over the first n positions."""
+    g = q.shape[0] // k.shape[0]
+    K, V = (np.repeat(t.astype(np.float64), g, 0)[:, :n] for t in (k, v))
+    with np.errstate(all="ignore"):
+        s = np.einsum("hd,htd->ht", q.astype(np.float64), K) / np.sqrt(q.shape[1])
+        e = np.exp(s - s.max(1, keepdims=True))
+        p = e / e.sum(1, keepdims=True)
+        return (p[:, :, None] * V).sum(1), p[-1]
+
+
+# the chunked kernel: one chunk (128 positions) and the first split (129), a
+# last chunk of one position, 16 / 32 / 64 column groups with idle lanes
+# (d = 4, 36, 100, 256), more heads than CUs, a masked tail; d = 30 and an
+# offset view stay on the general kernel
+@pytest.mark.parametrize("nq,nkv,d,seq,causal,shift", [
+    (12, 2, 128, 128, None, 0), (12, 2, 128, 129, None, 0), (28, 4, 128, 2049, None, 0),
+    (12, 2, 128, 512, 300, 0), (4, 4, 64, 1000, 999, 0), (3, 1, 4, 129, None, 0), (2, 1, 36, 161, 5, 0),
+    (2, 2, 100, 333, 200, 0), (7, 7, 256, 700, None, 0), (300, 1, 64, 257, None, 0),
+    (2, 1, 30, 300, None, 0), (2, 1, 64, 300, None, 1)])
+def test_gqa_chunks(nq, nkv, d, seq, causal, shift):
+    rng = np.random.default_rng(nq + d + seq)
+    q, k, v = (rng.standard_normal(s, dtype=np.float32)
+               for s in ((nq, d), (nkv, seq, d), (nkv, seq, d)))
+    kd = torch.zeros(k.size + shift, device=DEV)[shift:]
+    kd.copy_(dev(k).flatten())
+    y, probs = torch.zeros(nq * d, device=DEV), torch.full((seq,), 7.0, device=DEV)
+    myos.gqa_attn_f32(y, dev(q), kd, dev(v), probs, nq, nkv, d, seq, causal)
+    n = seq if causal is None else causal + 1
+    yr, pr = _gqa64(q, k, v, n)
+    # a score is a dot of d products within gamma_d |q||k| (< 2 gamma_d d for
+    # unit normals at these sizes) and moves its probability by that factor
+    tol = 8 * d * np.sqrt(d) * 2.0 ** -24 + seq * 2.0 ** -24
+    assert np.linalg.norm(host(y) - yr.ravel()) <= tol * np.linalg.norm(yr)
+    assert np.linalg.norm(host(probs)[:n] - pr) <= tol * np.linalg.norm(pr)
+    assert not host(probs)[n:].any()
+
+
+def test_gqa_chunks_non_finite():
+    # the row-wide definition, over 300 positions (several chunks): a NaN score
+    # takes its head; a chunk of -inf scores weighs nothing; all -inf is NaN; an
+    # infinite value under a zero probability is NaN in its column alone
+    nq, d, seq = 2, 64, 300
+    rng = np.random.default_rng(0)
+    q, k, v = (rng.standard_normal(s, dtype=np.float32) for s in ((nq, d), (nq, seq, d), (nq, seq, d)))
+    q[:, 0], k[:, :, 0] = 1.0, 0.0
+    cases = []
+    for name in ("nan", "chunk", "all", "value"):
+        k2, v2 = k.copy(), v.copy()
+        if name == "nan":
+            k2[0, 40, 3] = np.nan
+        elif name == "chunk":
+            k2[0, 0:64, 0] = -np.inf
+        elif name == "all":
+            k2[0, :, 0] = -np.inf
+        else:
+            k2[0, 64:128, 0] = -2000.0  # e^-250 next to the row's maximum: zero
+            v2[0, 70, 5] = np.inf
+        y, probs = torch.zeros(nq * d, device=DEV), torch.zeros(seq, device=DEV)
+        myos.gqa_attn_f32(y, dev(q), dev(k2), dev(v2), probs, nq, nq, d, seq)
+        got = host(y).reshape(nq, d)
+        with np.errstate(all="ignore"):
+            s = (np.einsum("hd,htd->ht", q, k2) / np.float32(np.sqrt(d))).astype(np.float32)
+            e = np.exp(s - np.nanmax(s, 1, keepdims=True), dtype=np.float32)
+            p = e / e.sum(1, keepdims=True)
+            ref = (p[:, :, None].astype(np.float64) * v2).sum(1)
+        assert np.array_equal(np.isnan(got), np.isnan(ref)), name
+        ok = ~np.isnan(ref)
+        assert np.allclose(got[ok], ref[ok], rtol=1e-4, atol=1e-5), name
