@@ -67,6 +67,12 @@ hipError_t launch_rmsnorm(float *y, const uint16_t *g, const float *x, size_t n,
                           hipStream_t s);
 hipError_t launch_rope_apply(float *x, size_t len, size_t head_dim, const float2 *cs,
                              hipStream_t s);
+// rope with the table passed by value (head_dim <= 2 * kRopeTabPairs)
+constexpr int kRopeTabPairs = 128;
+struct RopeTab {
+  float2 cs[kRopeTabPairs];
+};
+hipError_t launch_rope_apply_tab(float *x, size_t len, size_t head_dim, const RopeTab &tab, hipStream_t s);
 // floats of scratch launch_gqa_general needs (0: none)
 size_t gqa_scratch_floats(const float *y, const float *q, const float *k, const float *v, int nq, int d,
                           int seq, int mask, size_t query_pos);

@@ -157,15 +157,24 @@ int myos_rope_f32_inplace(float *x, size_t len, uint32_t position, size_t head_d
   if (head_dim == 0 || head_dim % 2 != 0) return MYOS_E_SHAPE;
   if (len == 0 || len % head_dim != 0) return MYOS_E_SHAPE;
   const size_t half = head_dim / 2;
-  std::vector<float2> cs(half);
   const float posf = (float)position;
-  for (size_t p = 0; p < half; p++) {
-    const float e = (float)(2 * p) / (float)head_dim;
-    const float inv = 1.0f / powf(theta, e);
-    const float ang = posf * inv;
-    cs[p] = make_float2(cosf(ang), sinf(ang));
-  }
+  auto fill = [&](float2 *cs) {
+    for (size_t p = 0; p < half; p++) {
+      const float e = (float)(2 * p) / (float)head_dim;
+      const float inv = 1.0f / powf(theta, e);
+      const float ang = posf * inv;
+      cs[p] = make_float2(cosf(ang), sinf(ang));
+    }
+  };
   hipStream_t s = S(stream);
+  if (half <= (size_t)kRopeTabPairs) {
+    RopeTab tab;
+    fill(tab.cs);
+    return hip_status(launch_rope_apply_tab(x, len, head_dim, tab, s));
+  }
+  // wider heads: a device copy of the table
+  std::vector<float2> cs(half);
+  fill(cs.data());
   float2 *dcs = nullptr;
   if (hipMallocAsync((void **)&dcs, half * sizeof(float2), s) != hipSuccess) return MYOS_E_HIP;
   hipError_t e = hipMemcpyAsync(dcs, cs.data(), half * sizeof(float2), hipMemcpyHostToDevice, s);

@@ -347,3 +347,15 @@ def test_gqa_chunks_non_finite():
         assert np.array_equal(np.isnan(got), np.isnan(ref)), name
         ok = ~np.isnan(ref)
         assert np.allclose(got[ok], ref[ok], rtol=1e-4, atol=1e-5), name
+
+
+# the table rides in the launch's arguments up to 128 pairs and is copied to the
+# device beyond; both must give the oracle's bits' values
+@pytest.mark.parametrize("d,heads", [(2, 3), (128, 12), (254, 2), (256, 2), (258, 2), (512, 1)])
+def test_rope_table_sizes(d, heads):
+    x0 = np.random.default_rng(d).standard_normal(heads * d, dtype=np.float32)
+    _, ref = oracle.rope_f32_inplace(x0, 77, d, THETA)
+    x = dev(x0)
+    myos.rope_f32_inplace(x, 77, d, THETA)
+    # the products may contract into fmas: one rounding of each term apart
+    assert np.max(np.abs(host(x) - ref)) <= 4 * 2.0 ** -24 * np.max(np.abs(x0))
