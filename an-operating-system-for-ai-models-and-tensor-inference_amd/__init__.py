@@ -165,6 +165,18 @@ def make_shape(hidden, num_q_heads, num_kv_heads, head_dim, intermediate, vocab,
 
 # ---------------------------------------------------------------- op tier ----
 
+# torch is imported by the first op call; model programs without torch never do
+_torch = _f32_dtype = _w16_dtypes = None
+
+
+def _load_torch():
+    global _torch, _f32_dtype, _w16_dtypes
+    import torch
+    _f32_dtype = torch.float32
+    _w16_dtypes = (torch.bfloat16, torch.int16, torch.uint16)
+    _torch = torch
+
+
 def _dev(t, name):
     """(pointer, element count) of a contiguous GPU tensor."""
     if t is None:
@@ -173,28 +185,32 @@ def _dev(t, name):
         raise ValueError(f"{name} must be a GPU tensor")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
-    return C.c_void_p(t.data_ptr()), t.numel()
+    return t.data_ptr(), t.numel()
 
 
 def _w16(t, name):
-    import torch
-    if t.dtype not in (torch.bfloat16, torch.int16, torch.uint16):
+    if _torch is None:
+        _load_torch()
+    if t.dtype not in _w16_dtypes:
         raise ValueError(f"{name} must hold BF16 bit patterns (bfloat16/int16/uint16)")
     return _dev(t, name)
 
 
 def _f32(t, name):
-    import torch
-    if t.dtype != torch.float32:
+    if _torch is None:
+        _load_torch()
+    if t.dtype != _f32_dtype:
         raise ValueError(f"{name} must be float32")
     return _dev(t, name)
 
 
 def _stream(stream):
-    import torch
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return C.c_void_p(stream.cuda_stream)
+        if _torch is None:
+            _load_torch()
+        # the handle torch.cuda.current_stream() wraps, without building the wrapper
+        return _torch._C._cuda_getCurrentRawStream(_torch.cuda.current_device())
+    return stream.cuda_stream
 
 
 def gemv_bf16(y, w, x, m, k, stream=None):

@@ -932,7 +932,7 @@ __global__ void rope_apply_tab_kernel(float *x, size_t len, int half, RopeTab ta
 // (o[d], max, sum) in part and gqa_merge_kernel combines them. K and V are read
 // in 16-byte lane loads by every CU the chunks fill, where the one-workgroup-
 // per-head kernel walks each K row in a single lane: 12 q / 2 kv heads of 128,
-// 2304 positions, 776 -> 31 us per call (most of it then host work).
+// 2304 positions, 776 -> 16 us per call.
 constexpr int kGqaThreads = 512, kGqaMaxChunk = 1024;
 
 template <int NJ>

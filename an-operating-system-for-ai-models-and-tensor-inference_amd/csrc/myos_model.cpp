@@ -32,6 +32,7 @@
 
 #include "../../include/myos_hip.h"
 #include "myos_internal.h"
+#include "myos_scratch.h"
 #include "myos_safetensors.h"
 
 using namespace myos;
@@ -649,6 +650,7 @@ void myos_model_close(myos_model *m) {
   if (m->trace) (void)hipFree(m->trace);
   if (m->host_state) (void)hipHostFree(m->host_state);
   if (m->stream) (void)hipStreamDestroy(m->stream);
+  op_scratch_trim();
   delete m;
 }
 

@@ -9,6 +9,7 @@
 
 #include "../../include/myos_hip.h"
 #include "myos_internal.h"
+#include "myos_scratch.h"
 
 using namespace myos;
 
@@ -85,20 +86,15 @@ int myos_gemm_bf16(float *y, size_t y_len, const uint16_t *w, size_t w_len, cons
   if (k == 0) return hip_status(launch_fill_zero(y, y_need, S(stream)));
   if (batch > INT32_MAX || m > INT32_MAX || k > INT32_MAX) return MYOS_E_SHAPE;
   hipStream_t s = S(stream);
-  uint16_t *hi = nullptr, *lo = nullptr;
-  if (hipMallocAsync((void **)&hi, x_need * 2, s) != hipSuccess) return MYOS_E_HIP;
-  if (hipMallocAsync((void **)&lo, x_need * 2, s) != hipSuccess) {
-    (void)hipFreeAsync(hi, s);
-    return MYOS_E_HIP;
-  }
-  // partials of the K splits (none when the grid already fills the device)
-  const size_t wsf = gemm_ws_floats((int)batch, (int)m, (int)k);
-  float *ws = nullptr;
-  if (wsf && hipMallocAsync((void **)&ws, wsf * 4, s) != hipSuccess) {
-    (void)hipFreeAsync(hi, s);
-    (void)hipFreeAsync(lo, s);
-    return MYOS_E_HIP;
-  }
+  // the bf16 hi / lo planes of X and the partials of the K splits (none when
+  // the grid already fills the device)
+  auto align256 = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  if (x_need > SIZE_MAX / 8) return MYOS_E_HIP;
+  const size_t plane = align256(x_need * 2), wsf = gemm_ws_floats((int)batch, (int)m, (int)k);
+  OpScratch scr(2 * plane + wsf * 4, s);
+  if (!scr.ok()) return MYOS_E_HIP;
+  uint16_t *hi = (uint16_t *)scr.get(), *lo = hi + plane / 2;
+  float *ws = wsf ? (float *)((uint8_t *)scr.get() + 2 * plane) : nullptr;
   hipError_t e = launch_split_rows(x, x_need, hi, lo, s);
   if (e == hipSuccess) {
     GemmArgs g{};
@@ -114,10 +110,8 @@ int myos_gemm_bf16(float *y, size_t y_len, const uint16_t *w, size_t w_len, cons
     e = launch_gemm(g, EPI_STORE, s);
     if (e == hipSuccess) e = launch_gemm_nan_repair(y, w, x, (int)batch, (int)m, (int)k, s);
   }
-  hipError_t f1 = hipFreeAsync(hi, s), f2 = hipFreeAsync(lo, s);
-  hipError_t f3 = ws ? hipFreeAsync(ws, s) : hipSuccess;
-  if (e == hipSuccess) e = f1 != hipSuccess ? f1 : f2 != hipSuccess ? f2 : f3;
-  return hip_status(e);
+  const hipError_t f = scr.done();
+  return hip_status(e != hipSuccess ? e : f);
 }
 
 // bf16.rs:147-158
@@ -208,12 +202,11 @@ int myos_gqa_attn_f32(float *y, size_t y_len, const float *q, size_t q_len, cons
   size_t scr_elems;
   if (!mul_ok(num_q_heads, seq_len, &scr_elems)) return MYOS_E_SHAPE;
   scr_elems = gqa_scratch_floats(y, q, k, v, (int)num_q_heads, (int)head_dim, (int)seq_len, mask, query_pos);
-  float *scr = nullptr;
-  if (scr_elems && hipMallocAsync((void **)&scr, scr_elems * sizeof(float), s) != hipSuccess)
-    return MYOS_E_HIP;
-  hipError_t e = launch_gqa_general(y, q, k, v, probs, scr, (int)num_q_heads, (int)num_kv_heads,
-                                    (int)head_dim, (int)seq_len, mask, query_pos, s);
-  hipError_t f = scr ? hipFreeAsync(scr, s) : hipSuccess;
+  OpScratch scr(scr_elems * sizeof(float), s);
+  if (!scr.ok()) return MYOS_E_HIP;
+  hipError_t e = launch_gqa_general(y, q, k, v, probs, (float *)scr.get(), (int)num_q_heads,
+                                    (int)num_kv_heads, (int)head_dim, (int)seq_len, mask, query_pos, s);
+  const hipError_t f = scr.done();
   return hip_status(e != hipSuccess ? e : f);
 }
 
@@ -308,8 +301,9 @@ int myos_greedy_token(uint32_t *out, const float *logits, size_t n, myos_stream_
   if (n == 0) return hip_status(hipMemsetAsync(out, 0, sizeof(uint32_t), s));
   if (n > UINT32_MAX) return MYOS_E_SHAPE;
   const int parts = argmax_parts(n);
-  float2 *part = nullptr;
-  if (hipMallocAsync((void **)&part, parts * sizeof(float2), s) != hipSuccess) return MYOS_E_HIP;
+  OpScratch scr(parts * sizeof(float2), s);
+  if (!scr.ok()) return MYOS_E_HIP;
+  float2 *part = (float2 *)scr.get();
   hipError_t e = launch_argmax_partial(logits, n, part, s);
   if (e == hipSuccess) {
     ArgmaxFinalArgs a;
@@ -319,7 +313,7 @@ int myos_greedy_token(uint32_t *out, const float *logits, size_t n, myos_stream_
     a.vocab = (uint32_t)n;
     e = launch_argmax_final(a, s);
   }
-  hipError_t f = hipFreeAsync(part, s);
+  const hipError_t f = scr.done();
   return hip_status(e != hipSuccess ? e : f);
 }
 

@@ -359,3 +359,37 @@ def test_rope_table_sizes(d, heads):
     myos.rope_f32_inplace(x, 77, d, THETA)
     # the products may contract into fmas: one rounding of each term apart
     assert np.max(np.abs(host(x) - ref)) <= 4 * 2.0 ** -24 * np.max(np.abs(x0))
+
+
+def test_scratch_streams_and_threads():
+    # calls that need scratch, from threads on their own streams and on one
+    # shared stream, growing and shrinking: each result is the one a lone call
+    # gives, bit for bit
+    import threading
+    rng = np.random.default_rng(5)
+    shapes = [(37, 640, 1536), (200, 1536, 640), (5, 70, 45)]
+    ins = [(dev(rand_w(rng, m, k), torch.int16),
+            dev(rng.standard_normal((b, k), dtype=np.float32))) for b, m, k in shapes]
+
+    def call(i):
+        b, m, k = shapes[i]
+        y = torch.zeros((b, m), device=DEV)
+        myos.gemm_bf16(y, *ins[i], b, m, k)
+        return y
+    want = [host(call(i)) for i in range(3)]
+    shared = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(t):
+        s = shared if t % 2 else torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            ys = [(i, call(i)) for _ in range(10) for i in range(3)]
+            s.synchronize()
+        bad.extend(i for i, y in ys if not np.array_equal(host(y), want[i]))
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
