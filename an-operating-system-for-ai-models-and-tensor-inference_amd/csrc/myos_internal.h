@@ -131,17 +131,17 @@ struct GemmArgs {
   float *ws;
   size_t ws_cap;               // floats at ws
   int kps;                     // set by the launcher: K steps per split
+  int n_base;                  // set by the launcher: first column of the launch
 };
-// Launch plan of the pipelined MFMA GEMM: tile shape (cfg 0..3 = 128 x 32,
-// 64, 128, 256) and K splits; cfg -1 takes the single-stage 128 x 64 kernel
-// (shapes the pipelined one does not take, and wide short-K projections)
+// Launch plan of the MFMA GEMM: tile shape and K splits (partials within
+// ws_cap floats); cfg -1 takes the single-stage 128 x 64 kernel (K % 64 != 0)
 struct GemmPlan {
   int cfg = -1;
   int splits = 1;
 };
-GemmPlan pf_plan(int M, int N, int K);
-// force every later plan to (cfg, splits); cfg < 0 restores the planner
-void gemm_force_plan(int cfg, int splits);
+GemmPlan gemm_plan(int M, int N, int K, size_t ws_cap);
+// the partial-buffer floats the plan uses when it may have any number
+size_t gemm_plan_ws_floats(int M, int N, int K);
 // the partial-buffer floats launch_gemm needs for this shape (0: one split)
 size_t gemm_ws_floats(int M, int N, int K);
 hipError_t launch_gemm(const GemmArgs &a, GemvEpi epi, hipStream_t s);

@@ -12,6 +12,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <initializer_list>
 
 #include "myos_internal.h"
 
@@ -1291,6 +1292,7 @@ __global__ void split_kernel(const float *X, size_t n, uint16_t *hi, uint16_t *l
 // mapping; the 32x32 result sits at row 8*(i/4) + 4*(l/32) + i%4, col l%32.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int GBM = 128, GBN = 64, GBK = 64, GLD = GBK + 8;  // LDS row pitch (bf16)
 
@@ -1520,394 +1522,355 @@ __global__ void __launch_bounds__(kBlock) gemm_mfma_kernel(GemmArgs a) {
   }
 }
 
-// ---- prefill GEMM with a two-stage LDS pipeline (K % 64 == 0) ---------------
+// ---- MFMA GEMM over direct-to-LDS loads (K % 64 == 0) -----------------------
 //
-// C[M,N] = (A_hi + A_lo)[M,K] . W[N,K]^T on v_mfma_f32_32x32x16_bf16. The
-// workgroup is WGM x WGN wavefronts; wave (wm, wn) owns a (32 MB) x (32 NB)
-// block of the (32 MB WGM) x (32 NB WGN) workgroup tile, MB x NB accumulators.
-// Per 64-wide K stage every thread loads its share of the A hi/lo and W rows
-// as 16-byte chunks (a wavefront load covers 8 rows x 128 B) into one of
-// three register sets, through buffer descriptors whose range ends at the
-// matrix, so rows past M or N read as zero; a set goes to one of two LDS
-// stages while the other stage is multiplied, one barrier per stage. Loads run
-// two stages ahead of their LDS store, and every stage issues its loads
-// unconditionally (a stage past the split reads out of range: zeros, no
-// traffic), so the compiler's wait before a store leaves the younger stages in
-// flight. An LDS row is the 128 B of one matrix row with chunk c at slot
-// c ^ (row & 7) ^ ((row >> 3) & 1): the 8 or 16 consecutive rows an MFMA
-// fragment read serves per LDS cycle (32 or 64 banks) hit distinct banks, and
-// so do the chunk stores. The next 16-wide K step's fragments are read from
-// LDS while the current step's MFMAs run.
-// LDS bytes per MFMA fall with MB and NB: (2 MB + NB) 1 KB fragments feed
-// 2 MB NB MFMAs (the hi and the lo term share each W fragment).
-template <int MB_, int NB_, int WGM_, int WGN_>
-struct PfCfg {
-  static constexpr int MB = MB_, NB = NB_, WGM = WGM_, WGN = WGN_;
-  static constexpr int NTH = 64 * WGM * WGN;
-  static constexpr int BM = 32 * MB * WGM, BN = 32 * NB * WGN;
-  static constexpr int ACH = BM * 8, WCH = BN * 8;  // 16-byte chunks per stage
-  static constexpr int ALD = (ACH + NTH - 1) / NTH, WLD = (WCH + NTH - 1) / NTH;
-  static constexpr int AL_OFF = ACH * 16, W_OFF = 2 * ACH * 16;
-  static constexpr int STAGE = (2 * ACH + WCH) * 16;
-  static constexpr int LDS = 2 * STAGE;
-  static constexpr int R = 3;  // register sets: loads run R - 1 stages ahead
+// C[M,N] = (A_hi + A_lo)[M,K] . W[N,K]^T. Operands go to LDS by
+// global_load_lds, with no registers or LDS stores in between, in a ring of
+// NST stages of KS columns. WM x WN x WK waves: wave (wm, wn, wk) multiplies
+// 16 MB rows by 16 NB columns over the stage's 32-wide K parts
+// [wk KP, (wk + 1) KP) with v_mfma_f32_16x16x32_bf16 (the hi and the lo term
+// share each W fragment); the WK partial tiles are added through LDS in order
+// at the end.
+// A stage's rows are KS * 2 bytes in 16-byte chunks; chunk c of row r sits at
+// slot c ^ dm_swz(r), so the eight rows that share an LDS cycle of a fragment
+// read hit distinct banks. A direct load writes lane order, so the swizzle is
+// in the lanes' global addresses.
+//
+// What bounds it, on MI355X, hi and lo products counted (us, kernel alone):
+// - many rows, wide tiles: the matrix cores. 2048 x 16384 x 1536 161, 2048 x
+//   3584 x 18944 in two splits 380 (1464 TFLOP/s), 8192 x 8192 x 4096 737
+//   (1490). The register-staged 128 x 256 kernel this replaces took 205, 460
+//   and 914: its LDS reads, LDS stores and MFMAs followed one another.
+// - up to 128 rows: the weight stream's latency. 128 x 17920 x 1536 is 25 us,
+//   of which 9 pass at K = 128; 8 x 37888 x 3584 reads its weights at 5.7 TB/s.
+template <int MB_, int NB_, int WM_, int WN_, int WK_, int KS_, int NST_, bool PP_ = false>
+struct DmCfg {
+  static constexpr int MB = MB_, NB = NB_, WM = WM_, WN = WN_, WK = WK_, KS = KS_, NST = NST_;
+  static constexpr bool PP = PP_;  // two wave groups take turns: see gemm_dma_kernel
+  static constexpr int NW = WM * WN * WK, NTH = 64 * NW, BM = 16 * MB * WM, BN = 16 * NB * WN;
+  static constexpr int CPR = KS / 8;               // chunks per row
+  static constexpr int RPI = 64 / CPR;             // rows per 1 KB load
+  static constexpr int AI = BM / RPI, WI = BN / RPI, NI = 2 * AI + WI;  // loads per stage
+  static constexpr int LPW = (NI + NW - 1) / NW;   // loads per wave and stage
+  static constexpr int STAGE = NI * 1024, TILE = BM * BN * 4;
+  static constexpr int EPL = WK > 1 ? WK * TILE : 0;  // partial tiles at the end
+  static constexpr int LDS = NST * STAGE > EPL ? NST * STAGE : EPL;
+  static constexpr int KP = KS / 32 / WK;          // 32-wide K parts per wave and stage
+  static_assert(BM % RPI == 0 && BN % RPI == 0 && LDS <= 160 * 1024 && KP >= 1 && NST >= 2, "tile");
+  static_assert(LPW * (NST - 2) < 63, "vmcnt");
 };
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t pf_rsrc(const uint16_t *base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc((void *)base, (short)0, (int)bytes, 0x00020000);
+template <int CPR>
+__device__ __forceinline__ int dm_swz(int r) {
+  return CPR == 4 ? (r >> 1) & 3 : r & 7;
 }
 
-// gemm_pf_kernel's QKV epilogue (bias, RoPE, q / K / V stores) by column
-// pairs: lane pair index pi takes columns (2j, 2j + 1) of tile row pi / (BN/2)
-// from the accumulator tile cs in LDS, so every lane works; a batch of pairs'
-// bias and RoPE reads goes out before its stores. REG 0 / 1 / 2: a full tile
-// of q / k / v columns with power-of-two head dims (shifts, no bounds or
-// region tests; KB: bf16 cache); REG 3: any tile, every test per pair. Same
-// arithmetic as gemm_store<EPI_QKV> for each element.
-template <class C, int REG, bool KB>
-__device__ __forceinline__ void qkv_pairs(const GemmArgs &a, const float *cs, int tid, int m0, int n0) {
-  // one batch of up to 32 pairs: with one wave per SIMD nothing hides a
-  // batch's read latency, so the reads go out together
-  constexpr int HB = C::BN / 2, NIT2 = C::BM * HB / C::NTH;
-  constexpr int EB2 = NIT2 <= 32 ? NIT2 : (NIT2 % 8 == 0 ? 8 : 1);
-  static_assert(C::BM * HB % C::NTH == 0, "whole epilogue iterations");
-  const int M = a.M, N = a.N, d = a.head_dim, half = d >> 1, qd = a.q_dim, qkd = a.q_dim + a.kv_dim;
-  const int lh = __builtin_ctz(half), ld = lh + 1;
-  for (int it0 = 0; it0 < NIT2; it0 += EB2) {
-    float2 bv[EB2], rv[EB2];
-#pragma unroll
-    for (int e = 0; e < EB2; e++) {
-      const int pi = tid + (it0 + e) * C::NTH;
-      const int row = REG < 3 ? m0 + pi / HB : min(m0 + pi / HB, M - 1);
-      const int col = REG < 3 ? n0 + 2 * (pi % HB) : min(n0 + 2 * (pi % HB), N - 2);
-      bv[e] = make_float2(a.bias[col], a.bias[col + 1]);
-      if (REG == 0 || REG == 1) {
-        const int rr = REG == 0 ? col : col - qd;
-        rv[e] = a.rope[(size_t)(a.start_pos + row) * half + ((rr >> 1) & (half - 1))];
-      } else if (REG == 3) {
-        const int rr = col < qd ? col : col - qd;  // v columns read an unused factor
-        rv[e] = a.rope[(size_t)(a.start_pos + row) * half + divmod_n(rr >> 1, half).y];
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < EB2; e++) {
-      const int pi = tid + (it0 + e) * C::NTH;
-      const int tr = pi / HB, tc = 2 * (pi % HB);
-      const int row = m0 + tr, col = n0 + tc;
-      if (REG == 3 && !(row < M && col < N)) continue;
-      const float2 yv = *(const float2 *)(cs + tr * C::BN + tc);
-      const float y0 = yv.x + bv[e].x, y1 = yv.y + bv[e].y;
-      const int pos = a.start_pos + row;
-      if (REG == 0) {
-        const int u = col >> 1;
-        const float o0 = y0 * rv[e].x - y1 * rv[e].y;
-        const float o1 = y1 * rv[e].x + y0 * rv[e].y;
-        float *qr = a.q_out + (size_t)row * qd + ((u >> lh) << ld) + (u & (half - 1));
-        qr[0] = o0;
-        qr[half] = o1;
-      } else if (REG == 1) {
-        const int u = (col - qd) >> 1;
-        const float o0 = y0 * rv[e].x - y1 * rv[e].y;
-        const float o1 = y1 * rv[e].x + y0 * rv[e].y;
-        const size_t base = ((size_t)(u >> lh) * a.max_seq + pos) * d + (u & (half - 1));
-        if (KB) {
-          ((uint16_t *)a.kc)[base] = f2bf(o0);
-          ((uint16_t *)a.kc)[base + half] = f2bf(o1);
-        } else {
-          ((float *)a.kc)[base] = o0;
-          ((float *)a.kc)[base + half] = o1;
-        }
-      } else if (REG == 2) {
-        const int rr = col - qkd;
-        const size_t base = ((size_t)(rr >> ld) * a.max_seq + pos) * d + (rr & (d - 1));
-        if (KB) {
-          *(uint32_t *)((uint16_t *)a.vc + base) = (uint32_t)f2bf(y0) | ((uint32_t)f2bf(y1) << 16);
-        } else {
-          *(float2 *)((float *)a.vc + base) = make_float2(y0, y1);
-        }
+// 64 lanes x 16 bytes from base + voff (per lane) into LDS at lds, lds + 16, ...
+// No destination register: completion is counted by vmcnt and waited for in
+// dm_wait. (The builtin would make the compiler drain every load before the
+// next LDS read.)
+__device__ __forceinline__ void dm_load(uint32_t lds, uint32_t voff, const void *base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base)
+               : "memory");
+}
+// this wave's loads but the last N have landed and its LDS reads are done;
+// after the barrier that holds for every wave
+template <int N>
+__device__ __forceinline__ void dm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// The epilogues on four consecutive columns (col % 4 == 0, in range) of one
+// row. Reads come first for a batch of them, then the stores (which may alias
+// the reads to the compiler).
+struct Epi4In {
+  float4 u, v;
+};
+template <int EPI>
+__device__ __forceinline__ Epi4In epi4_load(const GemmArgs &a, int row, int col) {
+  Epi4In in;
+  in.u = in.v = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (EPI == EPI_RESID) {
+    in.u = *(const float4 *)(a.y + (size_t)row * a.N + col);
+  } else if (EPI == EPI_QKV) {
+    in.u = *(const float4 *)(a.bias + col);
+    const int half = a.head_dim >> 1, rr = col < a.q_dim ? col : col - a.q_dim;
+    in.v = *(const float4 *)(a.rope + (size_t)(a.start_pos + row) * half + divmod_n(rr >> 1, half).y);
+  }
+  return in;
+}
+template <int EPI>
+__device__ __forceinline__ void epi4_store(const GemmArgs &a, int row, int col, f32x4 c, const Epi4In &in) {
+  if (EPI == EPI_STORE) {
+    *(f32x4 *)(a.y + (size_t)row * a.N + col) = c;
+  } else if (EPI == EPI_RESID) {
+    *(float4 *)(a.y + (size_t)row * a.N + col) =
+        make_float4(in.u.x + c[0], in.u.y + c[1], in.u.z + c[2], in.u.w + c[3]);
+  } else if (EPI == EPI_GU) {
+    const size_t o = (size_t)row * (a.N >> 1) + (col >> 1);
+    uint16_t h[2], l[2];
+    split2(silu(c[0]) * c[1], h, l);
+    split2(silu(c[2]) * c[3], h + 1, l + 1);
+    *(uint32_t *)(a.h_hi + o) = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
+    *(uint32_t *)(a.h_lo + o) = (uint32_t)l[0] | ((uint32_t)l[1] << 16);
+  } else {
+    const int d = a.head_dim, half = d >> 1, pos = a.start_pos + row, qkd = a.q_dim + a.kv_dim;
+    const float y0 = c[0] + in.u.x, y1 = c[1] + in.u.y, y2 = c[2] + in.u.z, y3 = c[3] + in.u.w;
+    auto pair = [&](uint16_t *p, float x, float y) { *(uint32_t *)p = (uint32_t)f2bf(x) | ((uint32_t)f2bf(y) << 16); };
+    if (col < qkd) {  // rotated pairs (y0, y1) and (y2, y3): columns p, p + 1 of both halves
+      const bool is_q = col < a.q_dim;
+      const int2 hp = divmod_n((is_q ? col : col - a.q_dim) >> 1, half);
+      const float a0 = y0 * in.v.x - y1 * in.v.y, b0 = y1 * in.v.x + y0 * in.v.y;
+      const float a1 = y2 * in.v.z - y3 * in.v.w, b1 = y3 * in.v.z + y2 * in.v.w;
+      if (is_q) {
+        float *qr = a.q_out + (size_t)row * a.q_dim + hp.x * d + hp.y;
+        *(float2 *)qr = make_float2(a0, a1);
+        *(float2 *)(qr + half) = make_float2(b0, b1);
       } else {
-        if (col < qkd) {
-          const bool is_q = col < qd;
-          const int2 hp = divmod_n((is_q ? col : col - qd) >> 1, half);
-          const float o0 = y0 * rv[e].x - y1 * rv[e].y;
-          const float o1 = y1 * rv[e].x + y0 * rv[e].y;
-          if (is_q) {
-            float *qr = a.q_out + (size_t)row * qd + hp.x * d + hp.y;
-            qr[0] = o0;
-            qr[half] = o1;
-          } else {
-            const size_t base = ((size_t)hp.x * a.max_seq + pos) * d + hp.y;
-            store_kv(a.kc, base, o0, a.kv_bf16);
-            store_kv(a.kc, base + half, o1, a.kv_bf16);
-          }
+        const size_t base = ((size_t)hp.x * a.max_seq + pos) * d + hp.y;
+        if (a.kv_bf16) {
+          pair((uint16_t *)a.kc + base, a0, a1);
+          pair((uint16_t *)a.kc + base + half, b0, b1);
         } else {
-          const int2 hj = divmod_n(col - qkd, d);
-          const size_t base = ((size_t)hj.x * a.max_seq + pos) * d + hj.y;
-          store_kv(a.vc, base, y0, a.kv_bf16);
-          store_kv(a.vc, base + 1, y1, a.kv_bf16);
+          *(float2 *)((float *)a.kc + base) = make_float2(a0, a1);
+          *(float2 *)((float *)a.kc + base + half) = make_float2(b0, b1);
         }
+      }
+    } else {
+      const int2 hj = divmod_n(col - qkd, d);
+      const size_t base = ((size_t)hj.x * a.max_seq + pos) * d + hj.y;
+      if (a.kv_bf16) {
+        pair((uint16_t *)a.vc + base, y0, y1);
+        pair((uint16_t *)a.vc + base + 2, y2, y3);
+      } else {
+        *(float4 *)((float *)a.vc + base) = make_float4(y0, y1, y2, y3);
       }
     }
   }
 }
+// CNT groups of four at (row[i], col[i]), those outside the matrix skipped.
+// EPI_STORE alone also takes any N and alignment (vec false: one by one).
+template <int EPI, int CNT>
+__device__ __forceinline__ void epi4_put(const GemmArgs &a, bool vec, float *ws, const int *row, const int *col,
+                                         const f32x4 *v) {
+  const int M = a.M, N = a.N;
+  if (EPI == EPI_STORE && !vec) {
+    float *y = ws ? ws : a.y;
+#pragma unroll
+    for (int i = 0; i < CNT; i++)
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (row[i] < M && col[i] + e < N) y[(size_t)row[i] * N + col[i] + e] = v[i][e];
+    return;
+  }
+  if (ws) {
+#pragma unroll
+    for (int i = 0; i < CNT; i++)
+      if (row[i] < M && col[i] < N) *(f32x4 *)(ws + (size_t)row[i] * N + col[i]) = v[i];
+    return;
+  }
+  Epi4In in[CNT];
+#pragma unroll
+  for (int i = 0; i < CNT; i++) in[i] = epi4_load<EPI>(a, min(row[i], M - 1), min(col[i], N - 4));
+#pragma unroll
+  for (int i = 0; i < CNT; i++)
+    if (row[i] < M && col[i] < N) epi4_store<EPI>(a, row[i], col[i], v[i], in[i]);
+}
 
-// TAIL: the launch covers the last gridDim.x * BN columns of N (a tail
-// launch after one over the first columns).
-template <class C, int EPI, bool TAIL = false>
-__global__ void __launch_bounds__(C::NTH) gemm_pf_kernel(GemmArgs a) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t pf_sm[];
-  constexpr int R = C::R;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave % C::WGM, wn = wave / C::WGM;
-  // Tile order. Workgroup L (in launch order) runs on XCD L % 8, and each XCD
-  // has its own L2. With 8 or more M tiles, XCD c takes the c-th contiguous
-  // run of tiles in an order that walks groups of 4 M tiles along N, so the
-  // workgroups resident on one XCD share their A and W panels: at 2048 rows
-  // the L2 hit rate goes from 44 % to 76 % (bit-identical output; each tile
-  // is computed the same way wherever it runs).
-  const int gx = gridDim.x, gy = gridDim.y, gxy = gx * gy;
-  int tn = blockIdx.x, tm = blockIdx.y, z = blockIdx.z;
+// a.n_base: first column of the launch (the launch covers a.n_base .. N - 1).
+template <class C, int EPI>
+__global__ void __launch_bounds__(C::NTH) gemm_dma_kernel(GemmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t dm_sm[];
+  constexpr int MB = C::MB, NB = C::NB, BN = C::BN, KS = C::KS, NST = C::NST, CPR = C::CPR;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % C::WM, wn = wave / C::WM % C::WN, wk = wave / (C::WM * C::WN);
+  // Tile order (workgroup L runs on XCD L % 8, each with its own L2): up to 7 M
+  // tiles, all those of one N tile on one XCD, which then reads the W panel
+  // once; from 8 on each XCD takes a contiguous run of an order that walks
+  // groups of 4 M tiles along N, so its L2 serves shared A and W panels (2048 x
+  // 16384 x 1536 on 8 M tiles: 168 -> 161 us).
+  const int gx = gridDim.x, gy = gridDim.y;
+  int tn, tm, z = blockIdx.z;
   if (gy >= 8) {
-    const int T = gxy * gridDim.z, L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+    const int gxy = gx * gy, T = gxy * gridDim.z, L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
     const int xc = L & 7, t = xc * (T >> 3) + min(xc, T & 7) + (L >> 3);
     z = t / gxy;
     const int t2 = t - z * gxy, g = t2 / (4 * gx), r = t2 - g * 4 * gx, gm = min(4, gy - 4 * g);
     tn = r / gm;
     tm = 4 * g + (r - tn * gm);
+  } else {
+    const int L = blockIdx.x + gx * blockIdx.y, gx8 = gx & ~7;
+    if (L < gx8 * gy) {
+      const int q = L >> 3;
+      tm = q % gy;
+      tn = q / gy * 8 + (L & 7);
+    } else {
+      const int q = L - gx8 * gy;
+      tm = q % gy;
+      tn = gx8 + q / gy;
+    }
   }
-  const int nb = TAIL ? a.N - gx * C::BN : 0;
-  const int n0 = nb + tn * C::BN, m0 = tm * C::BM;
+  const int n0 = a.n_base + tn * C::BN, m0 = tm * C::BM, S = gridDim.z;
   const int M = a.M, N = a.N, K = a.K;
-  const int nks = K >> 6, S = gridDim.z;
-  const int ks0 = (int)((long)z * nks / S), ks1 = (int)((long)(z + 1) * nks / S);
-  const int nst = ks1 - ks0;
-  // descriptors start at the tile's first row; rows past the matrix read 0
-  const __amdgpu_buffer_rsrc_t rah = pf_rsrc(a.a_hi + (size_t)m0 * K, (uint32_t)(M - m0) * K * 2);
-  const __amdgpu_buffer_rsrc_t ral = pf_rsrc(a.a_lo + (size_t)m0 * K, (uint32_t)(M - m0) * K * 2);
-  const __amdgpu_buffer_rsrc_t rw = pf_rsrc(a.w + (size_t)n0 * K, (uint32_t)(N - n0) * K * 2);
+  const int nks = K / KS;
+  const int ks0 = (int)((long)z * nks / S), ks1 = (int)((long)(z + 1) * nks / S), nst = ks1 - ks0;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)dm_sm;
 
-  u32x4 ra[R][C::ALD], rl[R][C::ALD], rb[R][C::WLD];
-  // stage ks into register set `set`; a stage past the split sits at byte
-  // offset 2^31 of each row, beyond every descriptor's range (< 2^31 bytes)
-  auto gload = [&](int set, int ks) {
-    const uint32_t kb = ks < ks1 ? (uint32_t)ks * 128u : 0x80000000u;
+  // load i of this wave covers RPI rows of one operand's stage; rows past the
+  // matrix are clamped (their results are not stored), and a wave with fewer
+  // loads repeats the last one, so every wave counts the same
+  uint32_t voff[C::LPW], ldst[C::LPW];
+  const uint16_t *src[C::LPW];
 #pragma unroll
-    for (int i = 0; i < C::ALD; i++) {
-      const int q = tid + i * C::NTH;
-      if (C::ACH % C::NTH == 0 || q < C::ACH) {
-        const int off = (int)((uint32_t)((q >> 3) * K * 2) + kb + (uint32_t)((q & 7) << 4));
-        ra[set][i] = __builtin_amdgcn_raw_buffer_load_b128(rah, off, 0, 0);
-        rl[set][i] = __builtin_amdgcn_raw_buffer_load_b128(ral, off, 0, 0);
-      }
-    }
+  for (int i = 0; i < C::LPW; i++) {
+    const int e = min(wave + i * C::NW, C::NI - 1);
+    const bool isw = e >= 2 * C::AI;
+    const int r = (isw ? e - 2 * C::AI : e % C::AI) * C::RPI + lane / CPR;
+    const int row = isw ? min(n0 + r, N - 1) : min(m0 + r, M - 1);
+    src[i] = isw ? a.w : e < C::AI ? a.a_hi : a.a_lo;
+    voff[i] = (uint32_t)row * (uint32_t)K * 2u + (uint32_t)(((lane % CPR) ^ dm_swz<CPR>(r)) * 16);
+    ldst[i] = lds0 + e * 1024;
+  }
+  auto gload = [&](int it) {  // stage it of the split (past the end: the last one again) into its slot
+    const size_t kb = (size_t)min(ks0 + it, ks1 - 1) * (KS * 2);
+    const uint32_t so = (uint32_t)(it % NST) * C::STAGE;
 #pragma unroll
-    for (int i = 0; i < C::WLD; i++) {
-      const int q = tid + i * C::NTH;
-      if (C::WCH % C::NTH == 0 || q < C::WCH) {
-        const int off = (int)((uint32_t)((q >> 3) * K * 2) + kb + (uint32_t)((q & 7) << 4));
-        rb[set][i] = __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0);
-      }
-    }
-  };
-  // the register set's chunks into LDS stage `st`: the thread's stores are
-  // numbered e = 0 .. NW - 1 (A hi, A lo, W) and part p of np takes those with
-  // e * np / NW == p
-  constexpr int NW = 2 * C::ALD + C::WLD;
-  auto swrite = [&](int set, int st, int p, int np) {
-    uint8_t *base = pf_sm + st * C::STAGE;
-#pragma unroll
-    for (int i = 0; i < C::ALD; i++) {
-      const int q = tid + i * C::NTH;
-      if (C::ACH % C::NTH == 0 || q < C::ACH) {
-        const int r = q >> 3, slot = ((q & 7) ^ (r & 7) ^ ((r >> 3) & 1)) << 4;
-        if ((2 * i) * np / NW == p) *(u32x4 *)(base + r * 128 + slot) = ra[set][i];
-        if ((2 * i + 1) * np / NW == p) *(u32x4 *)(base + C::AL_OFF + r * 128 + slot) = rl[set][i];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < C::WLD; i++) {
-      const int q = tid + i * C::NTH;
-      if (C::WCH % C::NTH == 0 || q < C::WCH) {
-        const int r = q >> 3, slot = ((q & 7) ^ (r & 7) ^ ((r >> 3) & 1)) << 4;
-        if ((2 * C::ALD + i) * np / NW == p) *(u32x4 *)(base + C::W_OFF + r * 128 + slot) = rb[set][i];
-      }
-    }
+    for (int i = 0; i < C::LPW; i++) dm_load(ldst[i] + so, voff[i], (const uint8_t *)src[i] + kb);
   };
 
-  f32x16 acc[C::MB][C::NB];
+  f32x4 acc[MB][NB];
 #pragma unroll
-  for (int i = 0; i < C::MB; i++)
+  for (int i = 0; i < MB; i++)
 #pragma unroll
-    for (int j = 0; j < C::NB; j++)
+    for (int j = 0; j < NB; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int l15 = lane & 15, lq = lane >> 4, sw = dm_swz<CPR>(l15);
+  const int arow = (wm * MB * 16 + l15) * (KS * 2), wrow = 2 * C::AI * 1024 + (wn * NB * 16 + l15) * (KS * 2);
+  // lane l of a fragment: row l % 16, K octet l / 16. W is the MFMA's row
+  // operand, so a lane ends with four consecutive columns of one row.
+  bf16x8 fw[NB], fh[MB], fl[MB];
+  auto frags = [&](int st, int kp) {
+    const uint8_t *base = dm_sm + st * C::STAGE;
+    const int slot = (((wk * C::KP + kp) * 4 + lq) ^ sw) * 16;
 #pragma unroll
-      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
-
-  const int arow = (wm * C::MB * 32 + (lane & 31)) * 128;
-  const int wrow = (wn * C::NB * 32 + (lane & 31)) * 128;
-  // the 64-wide stage in LDS stage `st`: 4 K steps of 16, each step's
-  // fragments read while the previous step's MFMAs run. After each step's
-  // MFMAs a quarter of register set `wset` goes to the other LDS stage (last
-  // read before the previous barrier), so the next stage's stores share the
-  // LDS with this stage's reads instead of stalling every wave after the
-  // barrier.
-  auto mult = [&](int st, int wset) {
-    const uint8_t *base = pf_sm + st * C::STAGE;
-    bf16x8 fh[2][C::MB], fl[2][C::MB], fw[2][C::NB];
-    auto ldfrag = [&](int buf, int ks) {
-      const int swz = ((2 * ks + (lane >> 5)) ^ (lane & 7) ^ ((lane >> 3) & 1)) << 4;
+    for (int j = 0; j < NB; j++)
+      fw[j] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(base + wrow + j * (32 * KS) + slot));
 #pragma unroll
-      for (int i = 0; i < C::MB; i++) {
-        fh[buf][i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(base + arow + i * 4096 + swz));
-        fl[buf][i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(base + C::AL_OFF + arow + i * 4096 + swz));
-      }
-#pragma unroll
-      for (int j = 0; j < C::NB; j++)
-        fw[buf][j] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(base + C::W_OFF + wrow + j * 4096 + swz));
-    };
-    ldfrag(0, 0);
-#pragma unroll
-    for (int ks = 0; ks < 4; ks++) {
-      const int b = ks & 1;
-      if (ks + 1 < 4) ldfrag(b ^ 1, ks + 1);
-#pragma unroll
-      for (int i = 0; i < C::MB; i++)
-#pragma unroll
-        for (int j = 0; j < C::NB; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fh[b][i], fw[b][j], acc[i][j], 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < C::MB; i++)
-#pragma unroll
-        for (int j = 0; j < C::NB; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fl[b][i], fw[b][j], acc[i][j], 0, 0, 0);
-      swrite(wset, st ^ 1, ks, 4);
-      // schedule of the step: one MFMA, then one of the next step's fragment
-      // reads, then one of the next stage's LDS stores, in turn (the reads
-      // stay ahead of their MFMAs, which the scheduler otherwise moves each
-      // read next to; against all reads first, then every MFMA: 2048-id
-      // prefill 14.98 -> 14.70 ms), and a fence at the step's end. In the
-      // stage's first step the global loads issued at the stage start go out
-      // two after each MFMA instead of in one burst (2048 ids a further
-      // 0.7 %; one or four after each MFMA, or two before it, no better).
-#pragma unroll
-      for (int g = 0; g < 2 * C::MB * C::NB; g++) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-        if (ks == 0) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);  // global loads
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-        __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // LDS write
-      }
-      __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < MB; i++) {
+      fh[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(base + arow + i * (32 * KS) + slot));
+      fl[i] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(base + C::AI * 1024 + arow + i * (32 * KS) + slot));
     }
   };
-
-  // stage s lives in register set s % R and LDS stage s & 1
+  auto mfmas = [&]() {
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[j], fh[i], acc[i][j], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[j], fl[i], acc[i][j], 0, 0, 0);
+  };
   if (nst > 0) {
-    gload(0, ks0);
-    swrite(0, 0, 0, 1);
 #pragma unroll
-    for (int s = 1; s < R; s++) gload(s, ks0 + s);
-  }
-  __syncthreads();
-  const int nfull = nst / R * R;
-  for (int it0 = 0; it0 < nfull; it0 += R) {
+    for (int s = 0; s < NST - 1; s++) gload(s);
+    int st = 0;
+    if constexpr (C::PP) {
+      // Waves 0-3 and 4-7 (one of each on every SIMD) run half a K part apart:
+      // while one group reads its fragments the other multiplies, so the LDS
+      // and the matrix cores are busy together (2048 x 16384 x 1536 on 256 x
+      // 256: 189 -> 168 us, 2048 x 3584 x 18944 450 -> 388). Every K part is a
+      // read phase, a barrier, a multiply phase, a barrier; the second group
+      // starts one barrier later. Stage it + 1 must have landed for everybody
+      // when the first group starts to read it: the first group waits for its
+      // share at the end of the last multiply phase of stage it, the second at
+      // the end of its last read phase. Stage it + NST - 1 takes the slot of
+      // stage it - 1, which the second group finished reading a barrier before.
+      static_assert(C::NW == 8, "two groups of four waves");
+      const bool late = wave >= 4;
+      dm_wait<C::LPW * (NST - 2)>();
+      if (late) dm_wait<63>();
+      for (int it = 0; it < nst; it++) {
 #pragma unroll
-    for (int u = 0; u < R; u++) {
-      const int it = it0 + u;
-      gload(u, ks0 + it + R);
-      mult(it & 1, (u + 1) % R);
-      __syncthreads();
+        for (int kp = 0; kp < C::KP; kp++) {
+          if (kp == 0) gload(it + NST - 1);
+          frags(st, kp);
+          __builtin_amdgcn_sched_barrier(0);
+          if (kp == C::KP - 1 && late) dm_wait<C::LPW * (NST - 2)>();
+          else dm_wait<63>();
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_setprio(1);
+          mfmas();
+          __builtin_amdgcn_s_setprio(0);
+          __builtin_amdgcn_sched_barrier(0);
+          if (kp == C::KP - 1 && !late) dm_wait<C::LPW * (NST - 2)>();
+          else dm_wait<63>();
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        st = st + 1 == NST ? 0 : st + 1;
+      }
+      if (!late) dm_wait<63>();
+    } else {
+      // the latency-bound tiles: each wave reads and multiplies as it can
+      for (int it = 0; it < nst; it++) {
+        // stage `it` has landed everywhere, and nobody reads stage it - 1 any
+        // more, whose slot the next load takes
+        dm_wait<C::LPW * (NST - 2)>();
+        gload(it + NST - 1);
+#pragma unroll
+        for (int kp = 0; kp < C::KP; kp++) {
+          frags(st, kp);
+          mfmas();
+        }
+        st = st + 1 == NST ? 0 : st + 1;
+      }
     }
   }
-#pragma unroll
-  for (int u = 0; u < R; u++) {
-    const int it = nfull + u;
-    if (it < nst) {
-      mult(it & 1, (u + 1) % R);
-      __syncthreads();
-    }
-  }
+  dm_wait<0>();
 
-  // the accumulator tile goes through LDS (free after the last stage's
-  // barrier), then each thread takes elements tid, tid + NTH, ... in row-major
-  // order: coalesced stores, and the epilogue's partner column (col ^ 1) is a
-  // plain LDS read
-  static_assert(C::BM * C::BN * 4 <= C::LDS, "accumulator tile exceeds the LDS stages");
-  float *cs = (float *)pf_sm;
+  float *ws = S > 1 ? a.ws + (size_t)z * M * N : nullptr;
+  const bool vec = EPI != EPI_STORE || ((N & 3) == 0 && (((uintptr_t)a.ws | (uintptr_t)a.y) & 15) == 0);
+  if constexpr (C::WK == 1) {
 #pragma unroll
-  for (int i = 0; i < C::MB; i++)
+    for (int i = 0; i < MB; i++) {
+      int row[NB], col[NB];
 #pragma unroll
-    for (int j = 0; j < C::NB; j++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int tr = wm * C::MB * 32 + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-        const int tc = wn * C::NB * 32 + j * 32 + (lane & 31);
-        cs[tr * C::BN + tc] = acc[i][j][e];
+      for (int j = 0; j < NB; j++) {
+        row[j] = m0 + (wm * MB + i) * 16 + l15;
+        col[j] = n0 + (wn * NB + j) * 16 + lq * 4;
       }
-  __syncthreads();
-  const bool split = S > 1;
-  float *ws = a.ws + (size_t)z * M * N;
-  if (EPI == EPI_GU && !split) {
-    // h = silu(gate) * up by column pairs (gate 2j, up 2j + 1), one pair per
-    // lane: every lane works and consecutive lanes write consecutive h
-    constexpr int HB = C::BN / 2;
-    for (int pi = tid; pi < C::BM * HB; pi += C::NTH) {
-      const int tr = pi / HB, tc = 2 * (pi % HB);
-      const int row = m0 + tr, col = n0 + tc;
-      if (row < M && col < N) {
-        const float2 gu = *(const float2 *)(cs + tr * C::BN + tc);
-        const size_t o = (size_t)row * (N >> 1) + (col >> 1);
-        split2(silu(gu.x) * gu.y, a.h_hi + o, a.h_lo + o);
-      }
+      epi4_put<EPI, NB>(a, vec, ws, row, col, acc[i]);
     }
-    return;
-  }
-  if (split || EPI == EPI_STORE || EPI == EPI_GU) {
-    for (int idx = tid; idx < C::BM * C::BN; idx += C::NTH) {
-      const int tr = idx / C::BN, tc = idx % C::BN;
-      const int row = m0 + tr, col = n0 + tc;
-      if (row < M && col < N) {
-        const float c = cs[idx];
-        if (split) ws[(size_t)row * N + col] = c;
-        else gemm_store<EPI>(a, row, col, c, cs[idx ^ 1]);
-      }
-    }
-    return;
-  }
-  if constexpr (EPI == EPI_QKV) {
-    // Decisions that are uniform for the tile are taken once here: a full
-    // tile whose columns are all q, all k or all v, with power-of-two head
-    // dims, runs a branch-free pair loop (see qkv_pairs).
-    const int half = a.head_dim >> 1, qd = a.q_dim, qkd = a.q_dim + a.kv_dim;
-    const bool fast = (half & (half - 1)) == 0 && m0 + C::BM <= M && n0 + C::BN <= N;
-    const int reg = !fast ? 3 : n0 + C::BN <= qd ? 0 : (n0 >= qd && n0 + C::BN <= qkd) ? 1 : n0 >= qkd ? 2 : 3;
-    const bool kb = a.kv_bf16 != 0;
-    switch (reg * 2 + (kb ? 1 : 0)) {
-      case 0: qkv_pairs<C, 0, false>(a, cs, tid, m0, n0); break;
-      case 1: qkv_pairs<C, 0, true>(a, cs, tid, m0, n0); break;
-      case 2: qkv_pairs<C, 1, false>(a, cs, tid, m0, n0); break;
-      case 3: qkv_pairs<C, 1, true>(a, cs, tid, m0, n0); break;
-      case 4: qkv_pairs<C, 2, false>(a, cs, tid, m0, n0); break;
-      case 5: qkv_pairs<C, 2, true>(a, cs, tid, m0, n0); break;
-      default: qkv_pairs<C, 3, false>(a, cs, tid, m0, n0); break;
-    }
-    return;
-  }
-  // the epilogues that read global memory: a batch of EB elements' reads
-  // first, then their stores
-  constexpr int NIT = C::BM * C::BN / C::NTH, EB = NIT % 8 == 0 ? 8 : 1;
-  static_assert(C::BM * C::BN % C::NTH == 0, "whole epilogue iterations");
-  for (int it0 = 0; it0 < NIT; it0 += EB) {
-    EpiIn in[EB];
+  } else {
+    // tile row r's 16-byte chunk c sits at slot c ^ (r & SW): the 16 rows a
+    // store covers spread over the banks
+    constexpr int TC = BN / 4, SW = TC % 8 == 0 ? 7 : 3;
+    static_assert(TC % (SW + 1) == 0, "swizzle stays in the row");
+    float *own = (float *)(dm_sm + wk * C::TILE);
 #pragma unroll
-    for (int e = 0; e < EB; e++) {
-      const int idx = tid + (it0 + e) * C::NTH;
-      const int row = m0 + idx / C::BN, col = n0 + idx % C::BN;
-      in[e] = gemm_epi_load<EPI>(a, min(row, M - 1), min(col, N - 1));  // clamped, unconditional
-    }
+    for (int i = 0; i < MB; i++)
 #pragma unroll
-    for (int e = 0; e < EB; e++) {
-      const int idx = tid + (it0 + e) * C::NTH;
-      const int row = m0 + idx / C::BN, col = n0 + idx % C::BN;
-      if (row < M && col < N) gemm_store_in<EPI>(a, row, col, cs[idx], cs[idx ^ 1], in[e]);
+      for (int j = 0; j < NB; j++) {
+        const int r = (wm * MB + i) * 16 + l15, c = (wn * NB + j) * 4 + lq;
+        *(f32x4 *)(own + r * BN + 4 * (c ^ (r & SW))) = acc[i][j];
+      }
+    __syncthreads();
+    constexpr int NG = C::BM * TC, EB = NG / C::NTH >= 4 ? 4 : 1;
+    for (int g0 = tid; g0 < NG; g0 += EB * C::NTH) {
+      int row[EB], col[EB];
+      f32x4 v[EB];
+#pragma unroll
+      for (int b = 0; b < EB; b++) {
+        const int g = g0 + b * C::NTH, r = min(g, NG - 1) / TC, c = min(g, NG - 1) % TC;
+        const float *p = (const float *)dm_sm + r * BN + 4 * (c ^ (r & SW));
+        v[b] = *(const f32x4 *)p;
+#pragma unroll
+        for (int w = 1; w < C::WK; w++) v[b] += *(const f32x4 *)(p + w * (C::TILE / 4));
+        row[b] = g < NG ? m0 + r : M;
+        col[b] = n0 + 4 * c;
+      }
+      epi4_put<EPI, EB>(a, vec, ws, row, col, v);
     }
   }
 }
@@ -3241,157 +3204,99 @@ hipError_t launch_split_rows(const float *X, size_t n, uint16_t *hi, uint16_t *l
 }
 
 // ---- GEMM launch plans ------------------------------------------------------
-// The pipelined kernel's tile shapes (M x N): 128 x 32, 128 x 64, 128 x 128,
-// 128 x 256. Wider tiles read fewer A bytes per weight byte (the A tile is
-// re-read by every N tile) and fewer LDS bytes per MFMA; narrower ones give
-// more workgroups when N is small.
-using PfT32 = PfCfg<1, 1, 4, 1>;
-using PfT64 = PfCfg<1, 2, 4, 1>;
-using PfT128 = PfCfg<2, 2, 2, 2>;
-using PfT256 = PfCfg<2, 4, 2, 2>;
-// 128 x 256 with eight waves (two per SIMD, 64 x 64 each): one wave's MFMAs
-// run while the other waits on LDS, which the four-wave 128 x 256 tile cannot
-using PfW256 = PfCfg<2, 2, 2, 4>;
-// 128 x 192 with eight waves (32 x 96 each): 8 N tiles of a 1536-wide
-// projection, so 16 M tiles x 2 splits fill the 256 CUs exactly
-using PfW192 = PfCfg<1, 3, 4, 2>;
-// Short prompts (at most 128 rows): 64-row tiles halve the activation bytes
-// each workgroup pulls per weight byte. 64 x 64 with four waves for the
-// narrow projections, 64 x 128 with eight waves for gate/up.
-using PfS64 = PfCfg<1, 1, 2, 2>;
-using PfS128 = PfCfg<1, 1, 2, 4>;
-// 64 x 160 with ten waves: a 17920-row gate/up at 65-128 rows is 224
-// workgroups, one round over the CUs, where the 64 x 128 tile's 280 put two
-// workgroups on 24 CUs
-using PfS160 = PfCfg<1, 1, 2, 5>;
-// 128 x 128 with eight waves (32 x 64 each): over 256 rows it takes the
-// 128 x 128 plans of the cost model (qkv 40.0 -> 32.4 us, o 38.0 -> 29.9 at
-// 2048 rows of the 1.5B shape)
-using PfW128 = PfCfg<1, 2, 4, 2>;
-constexpr int kPfCfgs = 10;
-constexpr int kPfPlanCfgs = 4;  // the cost model's candidates (the others are picked by shape)
-constexpr int kPfBN[kPfCfgs] = {PfT32::BN, PfT64::BN, PfT128::BN, PfT256::BN, PfW256::BN, PfW192::BN, PfS64::BN, PfS128::BN,
-                                PfS160::BN, PfW128::BN};
 constexpr int kCUs = 256;
 
-int g_force_cfg = -1, g_force_splits = 0;
+// gemm_dma_kernel's tiles, with the microseconds a 64-wide K step takes on one
+// CU (fitted to kernel times of this tile on MI355X over 8 to 8192 rows of the
+// 1.5B and 7B projections and of larger products). Eight waves with
+// alternating groups for the wide tiles; for few rows, tiles no taller than
+// the rows, whose time is the latency of their loads (there the alternation
+// measured slower: 7B gate/up at 128 rows on 128 x 160, 83 us against 91).
+using Dm256x256 = DmCfg<4, 8, 4, 2, 1, 32, 3, true>;
+using Dm128x512 = DmCfg<4, 8, 2, 4, 1, 32, 3, true>;
+using Dm128x384 = DmCfg<4, 6, 2, 4, 1, 32, 4, true>;
+using Dm128x128 = DmCfg<4, 4, 2, 2, 2, 64, 3, true>;
+using Dm128x96 = DmCfg<4, 3, 2, 2, 2, 64, 3, true>;
+using Dm128x160 = DmCfg<2, 10, 4, 1, 2, 64, 2>;
+using Dm128x80 = DmCfg<2, 5, 4, 1, 2, 64, 3>;
+using Dm128x64 = DmCfg<2, 4, 4, 1, 2, 64, 3>;
+using Dm64x80 = DmCfg<2, 5, 2, 1, 2, 64, 4>;
+using Dm64x64 = DmCfg<2, 4, 2, 1, 4, 128, 3, true>;
+using Dm64x128 = DmCfg<2, 4, 2, 2, 2, 64, 4, true>;
+using Dm32x80 = DmCfg<2, 5, 1, 1, 4, 128, 3>;
+using Dm32x64 = DmCfg<2, 4, 1, 1, 4, 128, 3>;
+using Dm16x80 = DmCfg<1, 5, 1, 1, 4, 128, 3>;
+using Dm16x64 = DmCfg<1, 4, 1, 1, 4, 128, 4>;
+struct DmTile {
+  int bm, bn, ks;
+  double t;
+};
+template <class C>
+constexpr DmTile dm_tile(double t) {
+  return {C::BM, C::BN, C::KS, t};
+}
+constexpr DmTile kDm[] = {dm_tile<Dm256x256>(2.35), dm_tile<Dm128x512>(2.5), dm_tile<Dm128x384>(2.05),
+                          dm_tile<Dm128x128>(0.8),  dm_tile<Dm128x96>(0.72), dm_tile<Dm128x160>(1.3),
+                          dm_tile<Dm128x80>(0.66),  dm_tile<Dm128x64>(0.6), dm_tile<Dm64x80>(0.53),
+                          dm_tile<Dm64x64>(0.45),   dm_tile<Dm64x128>(0.66), dm_tile<Dm32x80>(0.41),
+                          dm_tile<Dm32x64>(0.34),   dm_tile<Dm16x80>(0.26),  dm_tile<Dm16x64>(0.2)};
+constexpr int kDmTiles = sizeof(kDm) / sizeof(kDm[0]);
 
-// Tile shape and K splits for the pipelined kernel, from a cost model fitted
-// to measurements of this kernel on MI355X over the prefill shapes (1.5B and
-// 7B projections at 128 and 2048 rows). A workgroup is bound by what its CU
-// can pull from L2: about 64 outstanding 128-byte L2 requests at ~520 cycles
-// each, 14 B/clk, so a 64-wide K stage costs (A hi/lo 128 x 256 B + W
-// BN x 128 B) / 14 clocks; workgroups beyond one per CU run in further
-// rounds; K splits add their f32 partials written and read back at ~2 TB/s
-// and a reduction launch. Wider tiles re-read the A tile fewer times per
-// weight byte; split K fills the CUs when N has few tiles.
-GemmPlan pf_plan(int M, int N, int K) {
+// Microseconds of an M x N x K product on tile c in sp splits: launch, ramp and
+// output (f32 at about 3 TB/s), the rounds over the CUs (one workgroup each:
+// every tile's LDS is more than half a CU's), and for splits a reduction launch
+// and the partials written and read.
+static double dm_cost(int c, int M, int N, int K, int sp) {
+  const DmTile &d = kDm[c];
+  const long tiles = (long)((M + d.bm - 1) / d.bm) * ((N + d.bn - 1) / d.bn);
+  const long rounds = (tiles * sp + kCUs - 1) / kCUs, steps = (K / d.ks + sp - 1) / sp;
+  const double mn = (double)M * N * 4.0;
+  return 4.5 + rounds * (0.7 + steps * (d.ks / 64.0) * d.t) + (sp > 1 ? 3.2 + sp * mn * 0.45e-6 : mn / 3e6);
+}
+
+// The cheapest tile, whole or in as many K splits as fill one round of the CUs
+// and the partials' buffer (ws_cap floats) holds; cfg -1: K is not a multiple
+// of a 64-wide step (the single-stage kernel).
+GemmPlan gemm_plan(int M, int N, int K, size_t ws_cap) {
   GemmPlan best;
   if (K <= 0 || (K & 63) || M <= 0 || N <= 0) return best;
-  if (g_force_cfg >= 0) {
-    best.cfg = g_force_cfg;
-    best.splits = g_force_splits > 0 ? std::min(g_force_splits, K >> 6) : 1;
-    return best;
-  }
-  // Wide, short-K projections (gate/up: N >= 8192 rows of K <= 4096), and
-  // long-K ones (down) over many rows, take the eight-wave 128 x 256 tile.
-  // Measured per launch with the split reduction, weights from HBM (1.5B
-  // shapes): gate/up at 128 rows 48.3 us on the single-stage 128 x 64 kernel
-  // -> 45.4 (three splits), at 2048 rows 380 -> 326; down at 2048 rows 175
-  // (128 x 256, four waves, two splits) -> 140. The small projections and
-  // down at 128 rows stay on the cost model's choice (the eight-wave tiles
-  // measured no better there).
-  // Up to 128 rows, measured per launch with the split reduction (1.5B
-  // shapes, weights from HBM): gate/up without a split on the 64 x 160
-  // ten-wave tile where its grid fits one round (34.2 -> 26.7 us at 128
-  // rows), else on the 64 x 128 eight-wave tile (29.1 -> 23.5 us at 64 rows,
-  // 26.1 -> 19.7 at 32); where that grid would exceed ~1.25 rounds (the 7B
-  // gate/up, 592 workgroups) the 128 x 256 tile stays ahead.
-  if (N >= 8192 && K <= 4096) {
-    const long mt64 = (M + 63) / 64;
-    if (M > 64 && M <= 128 && mt64 * ((N + 159) / 160) <= kCUs) {
-      best.cfg = 8;
-      best.splits = 1;
-      return best;
-    }
-    if (M <= 128 && mt64 * ((N + 127) / 128) <= 320) {
-      best.cfg = 7;
-      best.splits = 1;
-      return best;
-    }
-    // (the 7B gate/up at 128 rows: 110.8 us with three splits, 107.5 with none)
-    best.cfg = 4;
-    best.splits = M > 128 && M <= 256 ? std::min(3, K >> 6) : 1;
-    return best;
-  }
-  // The other projections at up to 128 rows, except long-K ones wider than
-  // 2048 (the 7B down keeps the cost model's plan): a 64-row tile split so
-  // the grid fills one round over the CUs, the 64 x 64 four-wave tile or the
-  // 64 x 128 eight-wave one, whichever comes closer to 256 workgroups (the
-  // 64 x 64 on a tie). At 128 rows qkv 12.7 -> 11.0 us, o 11.6 -> 10.1,
-  // down 21.9 -> 19.7 (1.5B); 7B qkv 26.3 -> 22.6 (64 x 128, 3 splits), 7B
-  // o 21.5 -> 19.6 (64 x 64, 2 splits); at 32-64 rows qkv and o 1.8-3 us
-  // faster.
-  if (M <= 128 && (N <= 2048 || K <= 4096)) {
-    const long mt64 = (M + 63) / 64;
-    auto fill = [&](int bn, int *sp) {
-      const long tiles = mt64 * ((N + bn - 1) / bn);
-      *sp = (int)std::max(1L, std::min<long>({kCUs / tiles, 16L, (long)(K >> 6)}));
-      return tiles * *sp;
-    };
-    int s64 = 1, s128 = 1;
-    const long w64 = fill(64, &s64), w128 = fill(128, &s128);
-    if (w128 > w64 && w128 <= kCUs) {
-      best.cfg = 7;
-      best.splits = s128;
-    } else {
-      best.cfg = 6;
-      best.splits = s64;
-    }
-    return best;
-  }
-  if (M > 256 && N <= 4096 && K >= 4096) {
-    // the 128 x 192 tile when its two-split grid fits the CUs in one round
-    // (down at 2048 rows: 256 workgroups, 139 -> 121 us against 192 of the
-    // 128 x 256 tile)
-    const long t192 = ((M + 127) / 128) * (long)(N / 192);
-    best.cfg = N % 192 == 0 && 2 * t192 <= kCUs ? 5 : 4;
-    best.splits = 2;
-    return best;
-  }
-  const int nks = K >> 6;
-  const long mt = (M + 127) / 128;
   double best_t = 1e30;
-  for (int c = 0; c < kPfPlanCfgs; c++) {
-    const long tiles = mt * ((N + kPfBN[c] - 1) / kPfBN[c]);
-    const double stage = (32768.0 + 128.0 * kPfBN[c]) / 14.0;  // clocks per K stage
-    for (int sp = 1; sp <= std::min(nks, 64); sp++) {
-      const long rounds = (tiles * sp + kCUs - 1) / kCUs;
-      const int kst = (nks + sp - 1) / sp;
-      double t = rounds * (kst * stage + 1500.0) / 2400.0;  // us at 2.4 GHz
-      if (sp > 1) t += 2.0 * sp * (double)M * N * 4.0 / 2.0e6 + 1.0;
-      if (t < best_t - 1e-9) {
+  for (int c = 0; c < kDmTiles; c++) {
+    const DmTile &d = kDm[c];
+    if (K % d.ks) continue;
+    const long tiles = (long)((M + d.bm - 1) / d.bm) * ((N + d.bn - 1) / d.bn);
+    const long cap = std::min<long>({kCUs / tiles, 32L, (long)(K / std::max(d.ks, 64)), (long)(ws_cap / ((size_t)M * N))});
+    for (int sp : {1, (int)cap}) {
+      if (sp < 1 || (sp == 1 && best.cfg == c)) continue;
+      const double t = dm_cost(c, M, N, K, sp);
+      if (t < best_t) {
         best_t = t;
         best.cfg = c;
         best.splits = sp;
       }
     }
   }
-  if (M > 256 && best.cfg == 2) best.cfg = 9;  // the eight-wave 128 x 128 tile
   return best;
 }
 
-void gemm_force_plan(int cfg, int splits) {
-  g_force_cfg = cfg;
-  g_force_splits = splits;
-}
-
-// the pipelined kernel takes the shape: K stages of 64, 16-byte aligned
-// operands, 32-bit buffer ranges
-static bool pf_ok(const GemmArgs &a) {
-  return a.K > 0 && (a.K & 63) == 0 && a.M > 0 && a.N > 0 &&
-         (((uintptr_t)a.a_hi | (uintptr_t)a.a_lo | (uintptr_t)a.w) & 15) == 0 &&
-         (size_t)a.M * a.K * 2 < (1ull << 31) && (size_t)a.N * a.K * 2 < (1ull << 31);
+// gemm_dma_kernel takes the call: 16-byte aligned operands, 32-bit row offsets,
+// and for the epilogues on four columns at a time N and the head dim (so a
+// group stays in one head's q, k or v) multiples of 4 and aligned outputs
+template <int EPI>
+static bool dm_ok(const GemmArgs &a) {
+  auto aligned = [](uintptr_t n, std::initializer_list<const void *> ps) {
+    for (const void *p : ps)
+      if ((uintptr_t)p & (n - 1)) return false;
+    return true;
+  };
+  if (!aligned(16, {a.a_hi, a.a_lo, a.w}) || (size_t)a.M * a.K * 2 >= (1ull << 31) ||
+      (size_t)a.N * a.K * 2 >= (1ull << 31))
+    return false;
+  if (EPI == EPI_STORE) return true;
+  if ((a.N & 3) || !aligned(16, {a.ws})) return false;
+  if (EPI == EPI_RESID) return aligned(16, {a.y});
+  if (EPI == EPI_GU) return aligned(4, {a.h_hi, a.h_lo});
+  return (a.head_dim & 3) == 0 && aligned(16, {a.bias, a.rope, a.q_out, a.kc, a.vc});
 }
 
 int gemm_splits_old(int M, int N, int K) {
@@ -3408,28 +3313,64 @@ int gemm_splits_old(int M, int N, int K) {
   return (ksteps + kps - 1) / kps;
 }
 
-// Gate/up over many rows on the 128 x 256 tile: when the tiles fill some
-// rounds over the CUs and leave a partial round of at most half the CUs, the
-// N tiles that fill whole rounds run in one launch (returned: that many N
-// tiles) and the rest in a tail launch on 128 x 128 tiles, at most one round.
-// 2048 rows of the 1.5B gate/up: 1120 tiles = 4.375 rounds, 243 us ->
-// 1024 tiles (203-207 us), then 192 128 x 128 tiles (30 us), bit-identical.
-// (The tail as 96 x 2 half-K tiles took 28 us and their reduction 7.5.)
-// 0: one launch.
+// Gate/up over many rows: when the 256 x 256 tiles fill some rounds over the
+// CUs and leave a partial one, the N tiles of the whole rounds (returned: that
+// many) run in one launch and the columns left in a second, on the tile the
+// plan picks for them. 2048 rows of the 1.5B gate/up: 560 tiles, 2 whole rounds
+// 161 us and 1536 columns on 128 x 96 22 us, against 199 (estimated) on 752
+// tiles of 128 x 384. 0: one launch.
 static int gu_tail_plan(int M, int N, int K) {
-  static_assert(PfW256::BN % PfW128::BN == 0 && PfW256::BM == PfW128::BM, "tail tiles split the wide ones");
-  if (g_force_cfg >= 0 || K <= 0 || (K & 63) || M <= 0 || N % PfW256::BN) return 0;
-  const GemmPlan p = pf_plan(M, N, K);
-  if (p.cfg != 4 || p.splits != 1) return 0;
-  const long mt = (M + PfW256::BM - 1) / PfW256::BM, nt = N / PfW256::BN, tiles = mt * nt;
-  if (tiles <= kCUs || tiles % kCUs == 0) return 0;
-  const long nm = tiles / kCUs * kCUs / mt, tail = mt * (nt - nm);
-  return nm >= 1 && 2 * tail <= kCUs ? (int)nm : 0;
+  if (K <= 0 || (K & 63) || M <= 0 || N <= 0) return 0;
+  const DmTile &d = kDm[0];
+  const long mt = (M + d.bm - 1) / d.bm, nt = N / d.bn, tiles = mt * nt;
+  if (tiles <= kCUs || mt > kCUs) return 0;
+  const int nm = (int)(tiles / kCUs * kCUs / mt);
+  if (nm < 1 || (long)nm * d.bn >= N) return 0;
+  const GemmPlan whole = gemm_plan(M, N, K, 0), tail = gemm_plan(M, N - nm * d.bn, K, 0);
+  const double t = dm_cost(0, M, nm * d.bn, K, 1) + dm_cost(tail.cfg, M, N - nm * d.bn, K, 1);
+  return t < dm_cost(whole.cfg, M, N, K, 1) ? nm : 0;
+}
+
+// K splits that size the partials' buffer: a function of the shape alone, which
+// callers with fixed scratch are told (myos_gemm_bf16_noalloc_scratch), so it
+// does not move with the tiles above; plans stay within it. It came from tiles
+// of 128 x {32, 64, 128, 256} and 64 x {64, 128, 160}.
+static int gemm_scratch_splits(int M, int N, int K) {
+  if (K & 63) return 1;
+  const int nks = K >> 6;
+  const long mt64 = (M + 63) / 64, mt = (M + 127) / 128;
+  if (N >= 8192 && K <= 4096) return M > 128 && M <= 256 ? std::min(3, nks) : 1;
+  if (M <= 128 && (N <= 2048 || K <= 4096)) {
+    auto fill = [&](int bn, int *sp) {
+      const long tiles = mt64 * ((N + bn - 1) / bn);
+      *sp = (int)std::max(1L, std::min<long>({kCUs / tiles, 16L, (long)nks}));
+      return tiles * *sp;
+    };
+    int s64 = 1, s128 = 1;
+    const long w64 = fill(64, &s64), w128 = fill(128, &s128);
+    return w128 > w64 && w128 <= kCUs ? s128 : s64;
+  }
+  if (M > 256 && N <= 4096 && K >= 4096) return 2;
+  double best_t = 1e30;
+  int best = 1;
+  for (int bn : {32, 64, 128, 256}) {
+    const long tiles = mt * ((N + bn - 1) / bn);
+    const double stage = (32768.0 + 128.0 * bn) / 14.0;
+    for (int sp = 1; sp <= std::min(nks, 64); sp++) {
+      const long rounds = (tiles * sp + kCUs - 1) / kCUs;
+      double t = rounds * ((nks + sp - 1) / sp * stage + 1500.0) / 2400.0;
+      if (sp > 1) t += 2.0 * sp * (double)M * N * 4.0 / 2.0e6 + 1.0;
+      if (t < best_t - 1e-9) {
+        best_t = t;
+        best = sp;
+      }
+    }
+  }
+  return best;
 }
 
 size_t gemm_ws_floats(int M, int N, int K) {
-  const GemmPlan p = pf_plan(M, N, K);
-  const int sp = std::max(p.cfg >= 0 ? p.splits : 1, gemm_splits_old(M, N, K));
+  const int sp = std::max(gemm_scratch_splits(M, N, K), gemm_splits_old(M, N, K));
   return sp > 1 ? (size_t)sp * M * N : 0;
 }
 
@@ -3444,36 +3385,41 @@ static int gemm_plan_old(GemmArgs &a) {
   return splits;
 }
 
-// gx > 0: a grid gx tiles wide (the first gx tiles of N, or with TAIL the
-// last gx)
-template <class C, int EPI, bool TAIL = false>
-static hipError_t go_pf(const GemmArgs &a, int splits, hipStream_t s, int gx = 0) {
+// ncols > 0: only that many columns from a.n_base on
+template <class C, int EPI>
+static hipError_t go_dm(const GemmArgs &a, int splits, int ncols, hipStream_t s) {
   static bool attr_done = false;
-  const void *fn = (const void *)gemm_pf_kernel<C, EPI, TAIL>;
+  const void *fn = (const void *)gemm_dma_kernel<C, EPI>;
   if (!attr_done) {
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
     if (e != hipSuccess) return e;
     attr_done = true;
   }
-  dim3 grid(gx > 0 ? (unsigned)gx : nblk((size_t)a.N, C::BN), nblk((size_t)a.M, C::BM), splits);
   GemmArgs args = a;
   void *params[] = {&args};
-  return hipLaunchKernel(fn, grid, dim3(C::NTH), params, C::LDS, s);
+  return hipLaunchKernel(fn, dim3(nblk((size_t)ncols, C::BN), nblk((size_t)a.M, C::BM), splits), dim3(C::NTH), params,
+                         C::LDS, s);
 }
 
 template <int EPI>
-static hipError_t go_pf_cfg(const GemmArgs &a, int cfg, int splits, hipStream_t s) {
+static hipError_t go_dm_cfg(const GemmArgs &a, int cfg, int splits, int ncols, hipStream_t s) {
+  static_assert(kDmTiles == 15, "the order of kDm");
   switch (cfg) {
-    case 0: return go_pf<PfT32, EPI>(a, splits, s);
-    case 1: return go_pf<PfT64, EPI>(a, splits, s);
-    case 2: return go_pf<PfT128, EPI>(a, splits, s);
-    case 3: return go_pf<PfT256, EPI>(a, splits, s);
-    case 4: return go_pf<PfW256, EPI>(a, splits, s);
-    case 5: return go_pf<PfW192, EPI>(a, splits, s);
-    case 6: return go_pf<PfS64, EPI>(a, splits, s);
-    case 7: return go_pf<PfS128, EPI>(a, splits, s);
-    case 8: return go_pf<PfS160, EPI>(a, splits, s);
-    case 9: return go_pf<PfW128, EPI>(a, splits, s);
+    case 0: return go_dm<Dm256x256, EPI>(a, splits, ncols, s);
+    case 1: return go_dm<Dm128x512, EPI>(a, splits, ncols, s);
+    case 2: return go_dm<Dm128x384, EPI>(a, splits, ncols, s);
+    case 3: return go_dm<Dm128x128, EPI>(a, splits, ncols, s);
+    case 4: return go_dm<Dm128x96, EPI>(a, splits, ncols, s);
+    case 5: return go_dm<Dm128x160, EPI>(a, splits, ncols, s);
+    case 6: return go_dm<Dm128x80, EPI>(a, splits, ncols, s);
+    case 7: return go_dm<Dm128x64, EPI>(a, splits, ncols, s);
+    case 8: return go_dm<Dm64x80, EPI>(a, splits, ncols, s);
+    case 9: return go_dm<Dm64x64, EPI>(a, splits, ncols, s);
+    case 10: return go_dm<Dm64x128, EPI>(a, splits, ncols, s);
+    case 11: return go_dm<Dm32x80, EPI>(a, splits, ncols, s);
+    case 12: return go_dm<Dm32x64, EPI>(a, splits, ncols, s);
+    case 13: return go_dm<Dm16x80, EPI>(a, splits, ncols, s);
+    case 14: return go_dm<Dm16x64, EPI>(a, splits, ncols, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -3482,17 +3428,21 @@ static hipError_t go_pf_cfg(const GemmArgs &a, int cfg, int splits, hipStream_t 
 // EPI_STORE into the partials; returns the split count used in *splits_out.
 template <int EPI>
 static hipError_t gemm_main(GemmArgs &a, hipStream_t s, int *splits_out) {
-  const GemmPlan p = pf_plan(a.M, a.N, a.K);
-  if (p.cfg >= 0 && p.cfg < kPfCfgs && pf_ok(a) &&
-      (p.splits == 1 || (a.ws && a.ws_cap >= (size_t)p.splits * a.M * a.N))) {
+  const GemmPlan p = dm_ok<EPI>(a) ? gemm_plan(a.M, a.N, a.K, a.ws ? a.ws_cap : 0) : GemmPlan();
+  if (p.cfg >= 0) {
     *splits_out = p.splits;
-    return go_pf_cfg<EPI>(a, p.cfg, p.splits, s);
+    return go_dm_cfg<EPI>(a, p.cfg, p.splits, a.N, s);
   }
   const int splits = gemm_plan_old(a);
   *splits_out = splits;
   dim3 grid(nblk((size_t)a.N, GBN), nblk((size_t)a.M, GBM), splits);
   hipLaunchKernelGGL(gemm_mfma_kernel<EPI>, grid, dim3(kBlock), 0, s, a);
   return hipGetLastError();
+}
+
+size_t gemm_plan_ws_floats(int M, int N, int K) {
+  const GemmPlan p = gemm_plan(M, N, K, SIZE_MAX);
+  return p.splits > 1 ? (size_t)p.splits * M * N : 0;
 }
 
 hipError_t launch_gemm_resid_norm(const GemmArgs &args, const uint16_t *g, float eps,
@@ -3526,11 +3476,12 @@ template <int EPI>
 static hipError_t launch_gemm_epi(const GemmArgs &args, hipStream_t s) {
   GemmArgs a = args;
   if constexpr (EPI == EPI_GU) {
-    const int nm = gu_tail_plan(a.M, a.N, a.K);
-    if (nm > 0 && pf_ok(a)) {
-      hipError_t e = go_pf<PfW256, EPI_GU>(a, 1, s, nm);
+    const int nm = gu_tail_plan(a.M, a.N, a.K), nc = nm * kDm[0].bn;
+    if (nm > 0 && dm_ok<EPI>(a)) {
+      hipError_t e = go_dm_cfg<EPI_GU>(a, 0, 1, nc, s);
       if (e != hipSuccess) return e;
-      return go_pf<PfW128, EPI_GU, true>(a, 1, s, (a.N - nm * PfW256::BN) / PfW128::BN);
+      a.n_base = nc;
+      return go_dm_cfg<EPI_GU>(a, gemm_plan(a.M, a.N - nc, a.K, 0).cfg, 1, a.N - nc, s);
     }
   }
   int splits = 1;

@@ -369,10 +369,11 @@ int ensure_prefill(myos_model *m, size_t rows) {
   const size_t bt = align256(rows * 4);
   // K-split partials of the four projections
   const int R = (int)rows;
-  size_t wsf = gemm_ws_floats(R, (int)m->qkv_rows, (int)H);
-  wsf = std::max(wsf, gemm_ws_floats(R, (int)H, (int)Q));
-  wsf = std::max(wsf, gemm_ws_floats(R, (int)m->gu_rows, (int)H));
-  wsf = std::max(wsf, gemm_ws_floats(R, (int)H, (int)I));
+  size_t wsf = 0;
+  const size_t proj[4][2] = {{m->qkv_rows, H}, {H, Q}, {m->gu_rows, H}, {H, I}};
+  for (auto &nk : proj)
+    wsf = std::max({wsf, gemm_ws_floats(R, (int)nk[0], (int)nk[1]),
+                    gemm_plan_ws_floats(R, (int)nk[0], (int)nk[1])});
   // the attention's key-split partials use the same space (between GEMMs)
   if (m->s.head_dim == 128) wsf = std::max(wsf, attn_prefill_part_floats((int)m->s.num_q_heads, R, 4));
   const size_t bw = align256(wsf * 4);

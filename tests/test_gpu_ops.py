@@ -393,3 +393,29 @@ def test_scratch_streams_and_threads():
     for t in threads:
         t.join()
     assert not bad
+
+
+# gemm_bf16 over the direct-to-LDS tiles: each tile of the plan whole and (where
+# the plan splits it) in K splits, with row and column remainders: 64 x 80,
+# 16 x 64, 16 x 80, 32 x 64, 32 x 80, 64 x 64, 64 x 128, 128 x 64, 128 x 80,
+# 128 x 96, 128 x 128, 128 x 160, 128 x 384, 128 x 512, 256 x 256; N % 4 != 0
+# (scalar stores), one row, one K step, 8 or more M tiles (XCD runs)
+@pytest.mark.parametrize("batch,m,k", [
+    (2, 3515, 320), (34, 386, 1600), (66, 4269, 2112), (442, 458, 1664), (3, 671, 1536),
+    (244, 637, 2304), (39, 6293, 2368), (985, 350, 128), (90, 1510, 1856), (205, 1465, 768),
+    (140, 3545, 1536), (1012, 979, 384), (1, 3203, 2176), (757, 6394, 192), (21, 1535, 2176),
+    (305, 67, 2176), (527, 3087, 256), (513, 1240, 1600), (596, 3666, 512), (78, 2018, 2240),
+    (566, 5227, 64), (1207, 7514, 128), (2047, 8203, 448), (381, 37888, 192), (128, 20479, 320),
+    (2048, 1536, 8960), (1, 1, 64)])
+def test_gemm_tiles(batch, m, k):
+    g = torch.Generator(device=DEV).manual_seed(batch + m + k)
+    w = (torch.randn(m, k, generator=g, device=DEV) * 0.02).to(torch.bfloat16)
+    x = torch.randn(batch, k, generator=g, device=DEV)
+    y = torch.full((batch, m), float("nan"), device=DEV)
+    myos.gemm_bf16(y, w, x, batch, m, k)
+    ref = torch.mm(x.double(), w.double().t().contiguous())
+    mag = torch.mm(x.double().abs(), w.double().abs().t().contiguous())
+    # hi + lo keeps x to 2^-17 |x|; any summation order is within gamma_k, and
+    # MFMA accumulation may not round to nearest: 4 gamma_k
+    bound = (2.0 ** -17 + 4 * k * 2.0 ** -24) * mag
+    assert bool(((y.double() - ref).abs() <= bound).all())
