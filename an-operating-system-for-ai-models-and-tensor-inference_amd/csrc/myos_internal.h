@@ -57,9 +57,6 @@ hipError_t launch_attn_decode(const AttnDecodeArgs &a, hipStream_t s);
 
 // ---- small ops --------------------------------------------------------------
 hipError_t launch_fill_zero(float *y, size_t n, hipStream_t s);
-// recompute NaN outputs of Y[batch, m] = X W^T as the reference's f32 chain
-hipError_t launch_gemm_nan_repair(float *y, const uint16_t *w, const float *x, int batch, int m, int k,
-                                  hipStream_t s);
 hipError_t launch_add_bias(float *y, const uint16_t *b, size_t n, hipStream_t s);
 hipError_t launch_embed_gather(float *out, const uint16_t *table, size_t hidden,
                                const uint32_t *token_dev, uint32_t token_host, hipStream_t s);
@@ -115,6 +112,7 @@ hipError_t launch_split_rows(const float *X, size_t n, uint16_t *hi, uint16_t *l
 
 struct GemmArgs {
   const uint16_t *a_hi, *a_lo;  // [M, K] bf16 planes
+  const float *x;               // STORE by gemm_dma_kernel: [M, K] f32 instead
   const uint16_t *w;            // [N, K] bf16
   int M, N, K;
   float *y;                     // STORE: [M, N]; RESID: [M, N] +=
@@ -145,6 +143,11 @@ size_t gemm_plan_ws_floats(int M, int N, int K);
 // the partial-buffer floats launch_gemm needs for this shape (0: one split)
 size_t gemm_ws_floats(int M, int N, int K);
 hipError_t launch_gemm(const GemmArgs &a, GemvEpi epi, hipStream_t s);
+// the op tier's Y[M, N] = X W^T with the NaN outputs recomputed as the
+// reference's chain; hi / lo are used where gemm_needs_planes says so
+bool gemm_needs_planes(const float *x, const uint16_t *w, int M, int N, int K);
+hipError_t launch_gemm_op(float *y, const uint16_t *w, const float *x, int M, int N, int K, uint16_t *hi,
+                          uint16_t *lo, float *ws, size_t ws_cap, hipStream_t s);
 // EPI_RESID GEMM (y += A W^T) followed by the RMSNorm of y with gains g into
 // bf16 hi/lo planes, the split-K reduction and the norm in one pass when the
 // shape allows (else launch_gemm + launch_rmsnorm_rows_split)

@@ -1535,6 +1535,12 @@ __global__ void __launch_bounds__(kBlock) gemm_mfma_kernel(GemmArgs a) {
 // slot c ^ dm_swz(r), so the eight rows that share an LDS cycle of a fragment
 // read hit distinct banks. A direct load writes lane order, so the swizzle is
 // in the lanes' global addresses.
+// The op tier's product (EPI_STORE) on the few-row tiles takes A as the caller's
+// f32 rows: the stage holds them in the bytes of the two planes, and a fragment is
+// split into its hi and lo terms as it is read (37 x 8960 x 1536: 23.0 -> 15.7 us a
+// call with the split and NaN passes gone). On the tiles of 64 rows a wave the
+// splitting outlasts the other group's MFMAs (2048 x 3584 x 18944: kernel 387 ->
+// about 455 us), so they take X split by a pass before them.
 //
 // What bounds it, on MI355X, hi and lo products counted (us, kernel alone):
 // - many rows, wide tiles: the matrix cores. 2048 x 16384 x 1536 161, 2048 x
@@ -1547,6 +1553,7 @@ template <int MB_, int NB_, int WM_, int WN_, int WK_, int KS_, int NST_, bool P
 struct DmCfg {
   static constexpr int MB = MB_, NB = NB_, WM = WM_, WN = WN_, WK = WK_, KS = KS_, NST = NST_;
   static constexpr bool PP = PP_;  // two wave groups take turns: see gemm_dma_kernel
+  static constexpr bool XF = MB <= 2;  // EPI_STORE splits A itself
   static constexpr int NW = WM * WN * WK, NTH = 64 * NW, BM = 16 * MB * WM, BN = 16 * NB * WN;
   static constexpr int CPR = KS / 8;               // chunks per row
   static constexpr int RPI = 64 / CPR;             // rows per 1 KB load
@@ -1676,11 +1683,61 @@ __device__ __forceinline__ void epi4_put(const GemmArgs &a, bool vec, float *ws,
     if (row[i] < M && col[i] < N) epi4_store<EPI>(a, row[i], col[i], v[i], in[i]);
 }
 
+// eight consecutive f32 of a row as bf16 hi and lo terms (split2's values)
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split8(f32x4 a, f32x4 b, bf16x8 &hi, bf16x8 &lo) {
+  const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  uint32_t h[4], l[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const bf16x2 hv = __builtin_convertvector((f32x2{x[2 * e], x[2 * e + 1]}), bf16x2);
+    h[e] = __builtin_bit_cast(uint32_t, hv);
+    const bf16x2 lv = __builtin_convertvector((f32x2{x[2 * e] - bf_lo(h[e]), x[2 * e + 1] - bf_hi(h[e])}), bf16x2);
+    l[e] = __builtin_bit_cast(uint32_t, lv);
+  }
+  hi = __builtin_bit_cast(bf16x8, u32x4{h[0], h[1], h[2], h[3]});
+  lo = __builtin_bit_cast(bf16x8, u32x4{l[0], l[1], l[2], l[3]});
+}
+
+// n8 groups of eight: 16-byte loads and stores (2048 x 18944: 110 us one by one,
+// about 54 here)
+__global__ void __launch_bounds__(kBlock) split8_kernel(const float *X, size_t n8, uint16_t *hi, uint16_t *lo) {
+  const size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x;
+  if (i >= n8) return;
+  bf16x8 h, l;
+  split8(*(const f32x4 *)(X + 8 * i), *(const f32x4 *)(X + 8 * i + 4), h, l);
+  *(bf16x8 *)(hi + 8 * i) = h;
+  *(bf16x8 *)(lo + 8 * i) = l;
+}
+
+// y[row, col] of an EPI_STORE product as the reference's f32 chain. Every weight
+// meets the activation's bf16 hi and lo parts, and an infinite weight times a
+// zero lo part is NaN where the reference's chain (gemm_bf16.rs:337-378, left to
+// right from +0, each product rounded before it is added) gives +-inf; so an
+// output that is NaN is recomputed as that chain.
+__device__ float gemm_chain(const float *x, const uint16_t *w, int row, int col, int K) {
+  const uint16_t *wr = w + (size_t)col * K;
+  const float *xr = x + (size_t)row * K;
+  float acc = 0.f;
+  for (int j = 0; j < K; j++) acc = __fadd_rn(acc, __fmul_rn(bf16f(wr[j]), xr[j]));
+  return acc;
+}
+
+// an output this thread has stored
+__device__ __forceinline__ void gemm_repair(const GemmArgs &a, int row, int col) {
+  if (row >= a.M || col >= a.N) return;
+  float *y = a.y + (size_t)row * a.N + col;
+  if (__builtin_isnan(*y)) *y = gemm_chain(a.x, a.w, row, col, a.K);
+}
+
 // a.n_base: first column of the launch (the launch covers a.n_base .. N - 1).
 template <class C, int EPI>
 __global__ void __launch_bounds__(C::NTH) gemm_dma_kernel(GemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t dm_sm[];
   constexpr int MB = C::MB, NB = C::NB, BN = C::BN, KS = C::KS, NST = C::NST, CPR = C::CPR;
+  constexpr bool XF = EPI == EPI_STORE && C::XF;   // A is f32 rows of XCPR 16-byte chunks
+  constexpr int XCPR = 2 * CPR, XRPI = 64 / XCPR;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % C::WM, wn = wave / C::WM % C::WN, wk = wave / (C::WM * C::WN);
@@ -1720,22 +1777,31 @@ __global__ void __launch_bounds__(C::NTH) gemm_dma_kernel(GemmArgs a) {
   // matrix are clamped (their results are not stored), and a wave with fewer
   // loads repeats the last one, so every wave counts the same
   uint32_t voff[C::LPW], ldst[C::LPW];
-  const uint16_t *src[C::LPW];
+  int step[C::LPW];  // bytes of a row in a stage
+  const void *src[C::LPW];
 #pragma unroll
   for (int i = 0; i < C::LPW; i++) {
     const int e = min(wave + i * C::NW, C::NI - 1);
     const bool isw = e >= 2 * C::AI;
-    const int r = (isw ? e - 2 * C::AI : e % C::AI) * C::RPI + lane / CPR;
-    const int row = isw ? min(n0 + r, N - 1) : min(m0 + r, M - 1);
-    src[i] = isw ? a.w : e < C::AI ? a.a_hi : a.a_lo;
-    voff[i] = (uint32_t)row * (uint32_t)K * 2u + (uint32_t)(((lane % CPR) ^ dm_swz<CPR>(r)) * 16);
+    if (XF && !isw) {
+      const int r = e * XRPI + lane / XCPR;
+      src[i] = a.x;
+      voff[i] = (uint32_t)min(m0 + r, M - 1) * (uint32_t)K * 4u + (uint32_t)(((lane % XCPR) ^ dm_swz<XCPR>(r)) * 16);
+      step[i] = KS * 4;
+    } else {
+      const int r = (isw ? e - 2 * C::AI : e % C::AI) * C::RPI + lane / CPR;
+      const int row = isw ? min(n0 + r, N - 1) : min(m0 + r, M - 1);
+      src[i] = isw ? a.w : e < C::AI ? a.a_hi : a.a_lo;
+      voff[i] = (uint32_t)row * (uint32_t)K * 2u + (uint32_t)(((lane % CPR) ^ dm_swz<CPR>(r)) * 16);
+      step[i] = KS * 2;
+    }
     ldst[i] = lds0 + e * 1024;
   }
   auto gload = [&](int it) {  // stage it of the split (past the end: the last one again) into its slot
-    const size_t kb = (size_t)min(ks0 + it, ks1 - 1) * (KS * 2);
+    const size_t ks = (size_t)min(ks0 + it, ks1 - 1);
     const uint32_t so = (uint32_t)(it % NST) * C::STAGE;
 #pragma unroll
-    for (int i = 0; i < C::LPW; i++) dm_load(ldst[i] + so, voff[i], (const uint8_t *)src[i] + kb);
+    for (int i = 0; i < C::LPW; i++) dm_load(ldst[i] + so, voff[i], (const uint8_t *)src[i] + ks * step[i]);
   };
 
   f32x4 acc[MB][NB];
@@ -1744,13 +1810,31 @@ __global__ void __launch_bounds__(C::NTH) gemm_dma_kernel(GemmArgs a) {
 #pragma unroll
     for (int j = 0; j < NB; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int l15 = lane & 15, lq = lane >> 4, sw = dm_swz<CPR>(l15);
-  const int arow = (wm * MB * 16 + l15) * (KS * 2), wrow = 2 * C::AI * 1024 + (wn * NB * 16 + l15) * (KS * 2);
+  const int arow = (wm * MB * 16 + l15) * (KS * (XF ? 4 : 2)), wrow = 2 * C::AI * 1024 + (wn * NB * 16 + l15) * (KS * 2);
   // lane l of a fragment: row l % 16, K octet l / 16. W is the MFMA's row
   // operand, so a lane ends with four consecutive columns of one row.
   bf16x8 fw[NB], fh[MB], fl[MB];
   auto frags = [&](int st, int kp) {
     const uint8_t *base = dm_sm + st * C::STAGE;
     const int slot = (((wk * C::KP + kp) * 4 + lq) ^ sw) * 16;
+    if constexpr (XF) {
+      // A's reads go out first: its terms are split while W's arrive
+      const int c = ((wk * C::KP + kp) * 4 + lq) * 2, xs = dm_swz<XCPR>(l15);
+      const int s0 = (c ^ xs) * 16, s1 = ((c + 1) ^ xs) * 16;
+      f32x4 x0[MB], x1[MB];
+#pragma unroll
+      for (int i = 0; i < MB; i++) {
+        x0[i] = *(const f32x4 *)(base + arow + i * (64 * KS) + s0);
+        x1[i] = *(const f32x4 *)(base + arow + i * (64 * KS) + s1);
+      }
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+        fw[j] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(base + wrow + j * (32 * KS) + slot));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < MB; i++) split8(x0[i], x1[i], fh[i], fl[i]);
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < NB; j++)
       fw[j] = __builtin_bit_cast(bf16x8, *(const u32x4 *)(base + wrow + j * (32 * KS) + slot));
@@ -1830,6 +1914,7 @@ __global__ void __launch_bounds__(C::NTH) gemm_dma_kernel(GemmArgs a) {
   dm_wait<0>();
 
   float *ws = S > 1 ? a.ws + (size_t)z * M * N : nullptr;
+  bool bad = false;  // a NaN among this lane's EPI_STORE outputs
   const bool vec = EPI != EPI_STORE || ((N & 3) == 0 && (((uintptr_t)a.ws | (uintptr_t)a.y) & 15) == 0);
   if constexpr (C::WK == 1) {
 #pragma unroll
@@ -1841,7 +1926,16 @@ __global__ void __launch_bounds__(C::NTH) gemm_dma_kernel(GemmArgs a) {
         col[j] = n0 + (wn * NB + j) * 16 + lq * 4;
       }
       epi4_put<EPI, NB>(a, vec, ws, row, col, acc[i]);
+      if (EPI == EPI_STORE)
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) bad |= __builtin_isnan(acc[i][j][e]);
     }
+    if (EPI == EPI_STORE && S == 1 && bad)
+      for (int i = 0; i < MB; i++)
+        for (int j = 0; j < 4 * NB; j++)
+          gemm_repair(a, m0 + (wm * MB + i) * 16 + l15, n0 + (wn * NB + (j >> 2)) * 16 + lq * 4 + (j & 3));
   } else {
     // tile row r's 16-byte chunk c sits at slot c ^ (r & SW): the 16 rows a
     // store covers spread over the banks
@@ -1871,7 +1965,15 @@ __global__ void __launch_bounds__(C::NTH) gemm_dma_kernel(GemmArgs a) {
         col[b] = n0 + 4 * c;
       }
       epi4_put<EPI, EB>(a, vec, ws, row, col, v);
+      if (EPI == EPI_STORE)
+#pragma unroll
+        for (int b = 0; b < EB; b++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) bad |= __builtin_isnan(v[b][e]);
     }
+    if (EPI == EPI_STORE && S == 1 && bad)
+      for (int g = tid; g < NG; g += C::NTH)
+        for (int e = 0; e < 4; e++) gemm_repair(a, m0 + g / TC, n0 + 4 * (g % TC) + e);
   }
 }
 
@@ -1984,6 +2086,12 @@ __global__ void __launch_bounds__(kBlock) gemm_reduce4_kernel(GemmArgs a, int sp
     gemm_store_in<EPI>(a, row, col + 2, c.z, c.w, in[2]);
     gemm_store_in<EPI>(a, row, col + 3, c.w, c.z, in[3]);
   } else {
+    if (EPI == EPI_STORE && a.x) {
+      if (__builtin_isnan(c.x)) c.x = gemm_chain(a.x, a.w, row, col, a.K);
+      if (__builtin_isnan(c.y)) c.y = gemm_chain(a.x, a.w, row, col + 1, a.K);
+      if (__builtin_isnan(c.z)) c.z = gemm_chain(a.x, a.w, row, col + 2, a.K);
+      if (__builtin_isnan(c.w)) c.w = gemm_chain(a.x, a.w, row, col + 3, a.K);
+    }
     gemm_store<EPI>(a, row, col, c.x, c.y);
     gemm_store<EPI>(a, row, col + 1, c.y, c.x);
     gemm_store<EPI>(a, row, col + 2, c.z, c.w);
@@ -2005,6 +2113,10 @@ __global__ void __launch_bounds__(kBlock) gemm_reduce_kernel(GemmArgs a, int spl
   for (int z = 0; z < splits; z++) {
     c0 += a.ws[z * MN + off];
     if (two) c1 += a.ws[z * MN + off + 1];
+  }
+  if (EPI == EPI_STORE && a.x) {
+    if (__builtin_isnan(c0)) c0 = gemm_chain(a.x, a.w, row, col, a.K);
+    if (two && __builtin_isnan(c1)) c1 = gemm_chain(a.x, a.w, row, col + 1, a.K);
   }
   gemm_store<EPI>(a, row, col, c0, c1);
   if (two) gemm_store<EPI>(a, row, col + 1, c1, c0);
@@ -3024,27 +3136,18 @@ hipError_t launch_attn_decode(const AttnDecodeArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// The MFMA GEMM multiplies every weight by the activation's bf16 hi and lo
-// parts. An infinite weight times a zero lo part is NaN where the
-// reference's f32 chain (gemm_bf16.rs:337-378, bit-identical to the per-token
-// GEMV) gives +-inf, so a NaN output is recomputed here as that chain: left
-// to right from +0, each product rounded before it is added. Outputs that
-// are not NaN are left as they are; with finite weights and activations no
-// output is NaN and the pass only reads Y.
+// gemm_chain for the NaN outputs of the single-stage kernel; with finite weights
+// and activations no output is NaN and the pass only reads Y
 __global__ void gemm_nan_repair_kernel(float *y, const uint16_t *w, const float *x, int batch, int m, int k) {
   const size_t n = (size_t)batch * m;
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
     if (!__builtin_isnan(y[i])) continue;
     const size_t b = i / m, r = i - b * m;
-    const uint16_t *wr = w + r * k;
-    const float *xb = x + b * k;
-    float acc = 0.f;
-    for (int j = 0; j < k; j++) acc = __fadd_rn(acc, __fmul_rn(bf16f(wr[j]), xb[j]));
-    y[i] = acc;
+    y[i] = gemm_chain(x, w, (int)b, (int)r, k);
   }
 }
 
-hipError_t launch_gemm_nan_repair(float *y, const uint16_t *w, const float *x, int batch, int m, int k,
+static hipError_t launch_gemm_nan_repair(float *y, const uint16_t *w, const float *x, int batch, int m, int k,
                                   hipStream_t s) {
   const size_t n = (size_t)batch * m;
   if (!n) return hipSuccess;
@@ -3199,6 +3302,10 @@ hipError_t launch_rmsnorm_rows_split(const float *X, const uint16_t *g, float ep
 hipError_t launch_split_rows(const float *X, size_t n, uint16_t *hi, uint16_t *lo,
                              hipStream_t s) {
   if (!n) return hipSuccess;
+  if ((n & 7) == 0 && (((uintptr_t)X | (uintptr_t)hi | (uintptr_t)lo) & 15) == 0) {
+    hipLaunchKernelGGL(split8_kernel, dim3(nblk(n / 8, kBlock)), dim3(kBlock), 0, s, X, n / 8, hi, lo);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(split_kernel, dim3(nblk(n, 256)), dim3(256), 0, s, X, n, hi, lo);
   return hipGetLastError();
 }
@@ -3229,11 +3336,12 @@ using Dm16x80 = DmCfg<1, 5, 1, 1, 4, 128, 3>;
 using Dm16x64 = DmCfg<1, 4, 1, 1, 4, 128, 4>;
 struct DmTile {
   int bm, bn, ks;
+  bool xf;
   double t;
 };
 template <class C>
 constexpr DmTile dm_tile(double t) {
-  return {C::BM, C::BN, C::KS, t};
+  return {C::BM, C::BN, C::KS, C::XF, t};
 }
 constexpr DmTile kDm[] = {dm_tile<Dm256x256>(2.35), dm_tile<Dm128x512>(2.5), dm_tile<Dm128x384>(2.05),
                           dm_tile<Dm128x128>(0.8),  dm_tile<Dm128x96>(0.72), dm_tile<Dm128x160>(1.3),
@@ -3289,7 +3397,7 @@ static bool dm_ok(const GemmArgs &a) {
       if ((uintptr_t)p & (n - 1)) return false;
     return true;
   };
-  if (!aligned(16, {a.a_hi, a.a_lo, a.w}) || (size_t)a.M * a.K * 2 >= (1ull << 31) ||
+  if (!aligned(16, {a.x, a.a_hi, a.a_lo, a.w}) || (size_t)a.M * a.K * 2 >= (1ull << 31) ||
       (size_t)a.N * a.K * 2 >= (1ull << 31))
     return false;
   if (EPI == EPI_STORE) return true;
@@ -3443,6 +3551,40 @@ static hipError_t gemm_main(GemmArgs &a, hipStream_t s, int *splits_out) {
 size_t gemm_plan_ws_floats(int M, int N, int K) {
   const GemmPlan p = gemm_plan(M, N, K, SIZE_MAX);
   return p.splits > 1 ? (size_t)p.splits * M * N : 0;
+}
+
+// gemm_bf16's product. hi / lo: planes of M x K for the calls that need X split
+// (gemm_needs_planes); ws: gemm_ws_floats floats of partials.
+static bool gemm_op_direct(const GemmArgs &a) { return (a.K & 63) == 0 && dm_ok<EPI_STORE>(a); }
+bool gemm_needs_planes(const float *x, const uint16_t *w, int M, int N, int K) {
+  GemmArgs a{};
+  a.x = x;
+  a.w = w;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  return !gemm_op_direct(a) || !kDm[gemm_plan(M, N, K, gemm_ws_floats(M, N, K)).cfg].xf;
+}
+hipError_t launch_gemm_op(float *y, const uint16_t *w, const float *x, int M, int N, int K, uint16_t *hi,
+                          uint16_t *lo, float *ws, size_t ws_cap, hipStream_t s) {
+  GemmArgs g{};
+  g.x = x;
+  g.w = w;
+  g.M = M;
+  g.N = N;
+  g.K = K;
+  g.y = y;
+  g.ws = ws;
+  g.ws_cap = ws_cap;
+  if (gemm_needs_planes(x, w, M, N, K)) {
+    g.a_hi = hi;
+    g.a_lo = lo;
+    hipError_t e = launch_split_rows(x, (size_t)M * K, hi, lo, s);
+    if (e != hipSuccess) return e;
+  }
+  hipError_t e = launch_gemm(g, EPI_STORE, s);
+  // gemm_dma_kernel and the reduction of its splits look for NaN themselves
+  return e == hipSuccess && !gemm_op_direct(g) ? launch_gemm_nan_repair(y, w, x, M, N, K, s) : e;
 }
 
 hipError_t launch_gemm_resid_norm(const GemmArgs &args, const uint16_t *g, float eps,
