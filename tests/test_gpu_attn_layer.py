@@ -154,3 +154,31 @@ def test_errors_leave_residual_and_cache(tmp_path):
         # the same call at the cursor then succeeds and writes both
         assert call(0, 0, 4) == 0
         assert list(res) == [11, 15, 11, 15] and list(m.kv(0, 0, 0)[0]) == [1, 0]
+
+
+# decode attention at head_dim 128: a cache of up to 256 positions takes one
+# workgroup per query head, a longer one the chunk kernel; both from the first
+# position to the last, f32 and bf16 rows, against the oracle fed the same ids
+@pytest.mark.parametrize("kv", [myos.KV_F32, myos.KV_BF16])
+@pytest.mark.parametrize("max_seq,start", [(5, 0), (256, 0), (256, 249), (257, 250)])
+def test_decode_attention_rows(tmp_path, max_seq, start, kv):
+    from model_fixtures import random_map, write_safetensors
+    s = shape_dict(512, 4, 1, 128, 1536, 2048, 2, 1e-6)
+    t = random_map(s, seed=max_seq + start, std=0.05)
+    path = str(tmp_path / "m.safetensors")
+    write_safetensors(path, t)
+    shape = myos.make_shape(512, 4, 1, 128, 1536, 2048, 2)
+    ids = np.random.default_rng(start).integers(0, 2048, max_seq)
+    o = oracle.Model(s, t, max_seq, threads=4, kv_bf16=(kv == myos.KV_BF16))
+    # summation order only; bf16: a value near a rounding boundary may store as
+    # the neighbouring bf16 value (2^-8 of one element)
+    tol = 1e-4 if kv == myos.KV_F32 else 2e-3
+    with myos.Model.open(path, shape, kv, max_seq) as m:
+        if start:
+            m.prefill(ids[:start])
+            assert o.prefill(ids[:start]) == 0
+        for pos in range(start, min(max_seq, start + 8)):
+            m.forward_token(int(ids[pos]), pos)
+            assert o.forward_token(int(ids[pos]), pos) == 0
+            lg, lo = m.logits(), o.logits()
+            assert np.max(np.abs(lg - lo)) <= tol * np.max(np.abs(lo)), pos
