@@ -3159,7 +3159,10 @@ hipError_t pick_gemv(const GemvArgs &a, hipStream_t s, int *nparts) {
                    ((uintptr_t)a.x % 16) == 0 && (XM == X_PLAIN || ((uintptr_t)a.gamma % 8) == 0);
   if (!vec || a.k > 24576) return go_gemv_generic<XM, EPI>(a, s, nparts);
   const StreamPlan p = stream_plan(a.m, a.k);
-  if (p.grid > 0) return pick_stream<XM, EPI>(a, p, s, nparts);
+  // the epilogues that combine a team's rows two by two (gate and up, a RoPE pair)
+  // never take the streaming kernel's one-row batches (k > 4096)
+  const bool pairs = EPI == EPI_QKV || EPI == EPI_GU;
+  if (p.grid > 0 && (p.rb >= 2 || !pairs)) return pick_stream<XM, EPI>(a, p, s, nparts);
   const bool big = a.m >= 16384;
   if (nch <= 64 * 8) {
     const int cpt = (nch + 63) / 64;

@@ -380,3 +380,17 @@ def test_qwen15_prefill128_teacher_forced(qwen15):
     assert max_rel(k_g, k_o) < 1e-2 and max_rel(v_g, v_o) < 1e-2
     print("max logits rel err per step:", ["%.2e" % e for e in errs])
     g.close()
+
+
+def test_gate_up_rows_too_long_to_stream(tmp_path):
+    # 2 x 4096 gate/up rows of 4608 columns: long and many enough for the
+    # streaming GEMV, whose one-row batches cannot feed the gate/up pair epilogue
+    s = shape_dict(4608, 4, 1, 128, 4096, 512, 1, 1e-6)
+    t = random_map(s, seed=46, std=0.02)
+    g, o = open_pair(tmp_path, s, t, 8)
+    for pos, tok in enumerate((3, 141, 59)):
+        g.forward_token(tok, pos)
+        assert o.forward_token(tok, pos) == 0
+        assert max_rel(g.hidden(), o.hidden()) < 1e-4, pos
+        assert_logits_parity(g.logits(), o.logits(), f"step {pos}")
+    g.close()
