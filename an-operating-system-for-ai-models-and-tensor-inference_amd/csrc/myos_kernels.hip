@@ -3308,11 +3308,13 @@ hipError_t launch_rope_apply_tab(float *x, size_t len, size_t head_dim, const Ro
   return hipGetLastError();
 }
 
-// Positions per chunk of gqa_chunk_kernel: about two chunks per CU over all
-// heads, 32 to kGqaMaxChunk positions. Up to 128 positions one chunk per head
-// (no merge launch) is ahead.
-static int gqa_chunk(int nq, int seen) {
-  if (seen <= 128) return 128;
+// Positions per chunk of gqa_chunk_kernel: one chunk per head, with no scratch and
+// no merge launch, while a head's K and V are at most 1 MB and its scores fit LDS
+// (12 q / 2 kv heads of 128: 300 positions 11.9 -> 6.6 us a call, 1024 positions
+// 14.2 -> 11.6 among others and 25.5 -> 25.3 waited for alone); beyond, about two
+// chunks per CU over all heads, 32 to kGqaMaxChunk positions each.
+static int gqa_chunk(int nq, int d, int seen) {
+  if (seen <= kGqaMaxChunk && seen * d <= 128 * kGqaMaxChunk) return kGqaMaxChunk;
   const long per = (512 + nq - 1) / nq;  // chunks per head
   const long cp = (((seen + per - 1) / per) + 31) & ~31L;
   return (int)std::min<long>(std::max<long>(cp, 32), kGqaMaxChunk);
@@ -3329,7 +3331,7 @@ size_t gqa_scratch_floats(const float *y, const float *q, const float *k, const 
                           int seq, int mask, size_t query_pos) {
   if (!gqa_chunked(y, q, k, v, nq, d)) return (size_t)nq * seq;
   const int seen = mask && query_pos < (size_t)seq ? (int)query_pos + 1 : seq;
-  const int cp = gqa_chunk(nq, seen), nc = (int)(((long)seen + cp - 1) / cp);
+  const int cp = gqa_chunk(nq, d, seen), nc = (int)(((long)seen + cp - 1) / cp);
   return nc == 1 ? 0 : gqa_align4((size_t)nq * seq) + (size_t)nq * nc * (d + 4);
 }
 
@@ -3342,7 +3344,7 @@ hipError_t launch_gqa_general(float *y, const float *q, const float *k, const fl
     return hipGetLastError();
   }
   const int seen = mask && query_pos < (size_t)seq ? (int)query_pos + 1 : seq;
-  const int cp = gqa_chunk(nq, seen), nc = (int)(((long)seen + cp - 1) / cp);
+  const int cp = gqa_chunk(nq, d, seen), nc = (int)(((long)seen + cp - 1) / cp);
   float *part = scratch + (nc == 1 ? 0 : gqa_align4((size_t)nq * seq));
   const dim3 grid(nc, nq);
   if (d <= 64)

@@ -278,12 +278,13 @@ def _gqa64(q, k, v, n):
         return (p[:, :, None] * V).sum(1), p[-1]
 
 
-# the chunked kernel: one chunk (128 positions) and the first split (129), a
-# last chunk of one position, 16 / 32 / 64 column groups with idle lanes
+# the chunked kernel: one chunk (up to 1024 positions and 131072 values of K per
+# head) and the first split beyond, a last chunk of one position, 16 / 32 / 64 column groups with idle lanes
 # (d = 4, 36, 100, 256), more heads than CUs, a masked tail; d = 30 and an
 # offset view stay on the general kernel
 @pytest.mark.parametrize("nq,nkv,d,seq,causal,shift", [
-    (12, 2, 128, 128, None, 0), (12, 2, 128, 129, None, 0), (28, 4, 128, 2049, None, 0),
+    (12, 2, 128, 128, None, 0), (12, 2, 128, 1024, None, 0), (12, 2, 128, 1025, None, 0),
+    (2, 1, 256, 512, None, 0), (2, 1, 256, 513, None, 0), (28, 4, 128, 2049, None, 0),
     (12, 2, 128, 512, 300, 0), (4, 4, 64, 1000, 999, 0), (3, 1, 4, 129, None, 0), (2, 1, 36, 161, 5, 0),
     (2, 2, 100, 333, 200, 0), (7, 7, 256, 700, None, 0), (300, 1, 64, 257, None, 0),
     (2, 1, 30, 300, None, 0), (2, 1, 64, 300, None, 1)])
@@ -306,10 +307,10 @@ def test_gqa_chunks(nq, nkv, d, seq, causal, shift):
 
 
 def test_gqa_chunks_non_finite():
-    # the row-wide definition, over 300 positions (several chunks): a NaN score
+    # the row-wide definition, over 1100 positions (several chunks): a NaN score
     # takes its head; a chunk of -inf scores weighs nothing; all -inf is NaN; an
     # infinite value under a zero probability is NaN in its column alone
-    nq, d, seq = 2, 64, 300
+    nq, d, seq = 2, 64, 1100
     rng = np.random.default_rng(0)
     q, k, v = (rng.standard_normal(s, dtype=np.float32) for s in ((nq, d), (nq, seq, d), (nq, seq, d)))
     q[:, 0], k[:, :, 0] = 1.0, 0.0
