@@ -6,7 +6,7 @@
 // loads in flight per lane and to fuse the surrounding elementwise work
 // (RMSNorm prologue; bias + RoPE + KV-store, SwiGLU, residual and argmax
 // epilogues) so no activation round-trips through HBM between launches.
-// Prefill's projections run on MFMA (v_mfma_f32_32x32x16_bf16).
+// Prefill's projections run on MFMA (v_mfma_f32_16x16x32_bf16).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>

@@ -69,7 +69,7 @@ int myos_gemv_bf16(float *y, size_t y_len, const uint16_t *w, size_t w_len, cons
                    size_t x_len, size_t m, size_t k, myos_stream_t stream);
 
 /* gemm_bf16, crates/tensor_core/src/gemm_bf16.rs:51-110 (prefill projection).
- * Y[batch,m] = X[batch,k] W[m,k]^T on MFMA (v_mfma_f32_32x32x16_bf16) with X
+ * Y[batch,m] = X[batch,k] W[m,k]^T on MFMA (v_mfma_f32_16x16x32_bf16) with X
  * split into two BF16 terms (hi + lo) so the f32 activations keep ~16 mantissa
  * bits. The reference's caller-provided scratch is internal here. */
 int myos_gemm_bf16(float *y, size_t y_len, const uint16_t *w, size_t w_len, const float *x,
