@@ -125,7 +125,7 @@ struct GemmArgs {
   int kv_bf16, max_seq, q_dim, kv_dim, head_dim;
   // EPI_GU: writes h = silu(g)*u as hi/lo planes [M, N/2]
   uint16_t *h_hi, *h_lo;
-  // K-split partials [splits][M][N] f32 (gemm_ws_floats); null: one split
+  // K-split partials [splits][M][N] f32; null: one split
   float *ws;
   size_t ws_cap;               // floats at ws
   int kps;                     // set by the launcher: K steps per split
@@ -138,9 +138,13 @@ struct GemmPlan {
   int splits = 1;
 };
 GemmPlan gemm_plan(int M, int N, int K, size_t ws_cap);
-// the partial-buffer floats the plan uses when it may have any number
-size_t gemm_plan_ws_floats(int M, int N, int K);
-// the partial-buffer floats launch_gemm needs for this shape (0: one split)
+// partial-buffer floats that no plan for up to M rows exceeds: the model's products
+// are planned by their shape alone, and the need does not grow with the rows, so a
+// buffer sized by the longest prompt's own plan would not hold (or, capping the
+// plan, would change the sums of) a shorter one
+size_t gemm_ws_bound(int M, int N, int K);
+// the partial-buffer floats of the op tier's product (0: one split); a function of
+// the shape as well
 size_t gemm_ws_floats(int M, int N, int K);
 hipError_t launch_gemm(const GemmArgs &a, GemvEpi epi, hipStream_t s);
 // the op tier's Y[M, N] = X W^T with the NaN outputs recomputed as the

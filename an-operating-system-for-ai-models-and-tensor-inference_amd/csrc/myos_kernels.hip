@@ -3478,28 +3478,38 @@ static double dm_cost(int c, int M, int N, int K, int sp) {
   return 4.5 + rounds * (0.7 + steps * (d.ks / 64.0) * d.t) + (sp > 1 ? 3.2 + sp * mn * 0.45e-6 : mn / 3e6);
 }
 
-// The cheapest tile, whole or in as many K splits as fill one round of the CUs
-// and the partials' buffer (ws_cap floats) holds; cfg -1: K is not a multiple
-// of a 64-wide step (the single-stage kernel).
-GemmPlan gemm_plan(int M, int N, int K, size_t ws_cap) {
-  GemmPlan best;
-  if (K <= 0 || (K & 63) || M <= 0 || N <= 0) return best;
-  double best_t = 1e30;
+// The plans of a shape: every tile, whole and in as many K splits as fill one
+// round of the CUs and the partials' buffer (ws_cap floats) holds. A wide tile's
+// partials are 256 KB a CU, written after the loop, however short the splits make
+// the loop: at most 12 (200 x 3584 x 18944: 256 x 256 in 18 splits 66 + 11 us with
+// the reduction, 128 x 128 in 4 62 + 6).
+template <class F>
+static void each_plan(int M, int N, int K, size_t ws_cap, F f) {
   for (int c = 0; c < kDmTiles; c++) {
     const DmTile &d = kDm[c];
     if (K % d.ks) continue;
     const long tiles = (long)((M + d.bm - 1) / d.bm) * ((N + d.bn - 1) / d.bn);
-    const long cap = std::min<long>({kCUs / tiles, 32L, (long)(K / std::max(d.ks, 64)), (long)(ws_cap / ((size_t)M * N))});
-    for (int sp : {1, (int)cap}) {
-      if (sp < 1 || (sp == 1 && best.cfg == c)) continue;
-      const double t = dm_cost(c, M, N, K, sp);
-      if (t < best_t) {
-        best_t = t;
-        best.cfg = c;
-        best.splits = sp;
-      }
-    }
+    const long most = d.bm * d.bn < 256 * 256 ? 32 : 12;
+    const long cap = std::min<long>({kCUs / tiles, most, (long)(K / std::max(d.ks, 64)), (long)(ws_cap / ((size_t)M * N))});
+    f(c, 1);
+    if (cap > 1) f(c, (int)cap);
   }
+}
+
+// The cheapest; cfg -1: K is not a multiple of a 64-wide step (the single-stage
+// kernel).
+GemmPlan gemm_plan(int M, int N, int K, size_t ws_cap) {
+  GemmPlan best;
+  if (K <= 0 || (K & 63) || M <= 0 || N <= 0) return best;
+  double best_t = 1e30;
+  each_plan(M, N, K, ws_cap, [&](int c, int sp) {
+    const double t = dm_cost(c, M, N, K, sp);
+    if (t < best_t) {
+      best_t = t;
+      best.cfg = c;
+      best.splits = sp;
+    }
+  });
   return best;
 }
 
@@ -3593,6 +3603,27 @@ static int gemm_scratch_splits(int M, int N, int K) {
   return best;
 }
 
+// Within sixteen rows every tile keeps its count, and a plan's time only grows with
+// the rows: a plan that is slower at the first of them than another at the last is
+// never the cheapest.
+size_t gemm_ws_bound(int M, int N, int K) {
+  size_t need = 0;
+  for (long m = 1; m <= M; m++) {
+    const int sp = gemm_splits_old((int)m, N, K);
+    if (sp > 1) need = std::max(need, (size_t)sp * m * N);
+  }
+  if (K & 63) return need;
+  for (long lo = 1; lo <= M; lo += 16) {
+    const int hi = (int)std::min<long>(lo + 15, M);
+    double best = 1e30;
+    each_plan(hi, N, K, SIZE_MAX, [&](int c, int sp) { best = std::min(best, dm_cost(c, hi, N, K, sp)); });
+    each_plan((int)lo, N, K, SIZE_MAX, [&](int c, int sp) {
+      if (sp > 1 && dm_cost(c, (int)lo, N, K, sp) <= best) need = std::max(need, (size_t)sp * hi * N);
+    });
+  }
+  return need;
+}
+
 size_t gemm_ws_floats(int M, int N, int K) {
   const int sp = std::max(gemm_scratch_splits(M, N, K), gemm_splits_old(M, N, K));
   return sp > 1 ? (size_t)sp * M * N : 0;
@@ -3652,8 +3683,12 @@ static hipError_t go_dm_cfg(const GemmArgs &a, int cfg, int splits, int ncols, h
 // EPI_STORE into the partials; returns the split count used in *splits_out.
 template <int EPI>
 static hipError_t gemm_main(GemmArgs &a, hipStream_t s, int *splits_out) {
-  const GemmPlan p = dm_ok<EPI>(a) ? gemm_plan(a.M, a.N, a.K, a.ws ? a.ws_cap : 0) : GemmPlan();
+  // the op tier's product plans within the scratch its entry points state; the
+  // model's by their shape alone, in a buffer of gemm_ws_bound floats
+  const size_t cap = EPI != EPI_STORE ? SIZE_MAX : a.ws ? a.ws_cap : 0;
+  const GemmPlan p = dm_ok<EPI>(a) ? gemm_plan(a.M, a.N, a.K, cap) : GemmPlan();
   if (p.cfg >= 0) {
+    if (p.splits > 1 && (!a.ws || a.ws_cap < (size_t)p.splits * a.M * a.N)) return hipErrorInvalidValue;
     *splits_out = p.splits;
     return go_dm_cfg<EPI>(a, p.cfg, p.splits, a.N, s);
   }
@@ -3662,11 +3697,6 @@ static hipError_t gemm_main(GemmArgs &a, hipStream_t s, int *splits_out) {
   dim3 grid(nblk((size_t)a.N, GBN), nblk((size_t)a.M, GBM), splits);
   hipLaunchKernelGGL(gemm_mfma_kernel<EPI>, grid, dim3(kBlock), 0, s, a);
   return hipGetLastError();
-}
-
-size_t gemm_plan_ws_floats(int M, int N, int K) {
-  const GemmPlan p = gemm_plan(M, N, K, SIZE_MAX);
-  return p.splits > 1 ? (size_t)p.splits * M * N : 0;
 }
 
 // gemm_bf16's product. hi / lo: planes of M x K for the calls that need X split

@@ -367,13 +367,11 @@ int ensure_prefill(myos_model *m, size_t rows) {
   const size_t bx = align256(rows * H * 4), bq = align256(rows * Q * 4);
   const size_t ba = align256(rows * (H > Q ? H : Q) * 2), bh = align256(rows * I * 2);
   const size_t bt = align256(rows * 4);
-  // K-split partials of the four projections
+  // K-split partials of the four projections, for any prompt of up to `rows` ids
   const int R = (int)rows;
   size_t wsf = 0;
   const size_t proj[4][2] = {{m->qkv_rows, H}, {H, Q}, {m->gu_rows, H}, {H, I}};
-  for (auto &nk : proj)
-    wsf = std::max({wsf, gemm_ws_floats(R, (int)nk[0], (int)nk[1]),
-                    gemm_plan_ws_floats(R, (int)nk[0], (int)nk[1])});
+  for (auto &nk : proj) wsf = std::max(wsf, gemm_ws_bound(R, (int)nk[0], (int)nk[1]));
   // the attention's key-split partials use the same space (between GEMMs)
   if (m->s.head_dim == 128) wsf = std::max(wsf, attn_prefill_part_floats((int)m->s.num_q_heads, R, 4));
   const size_t bw = align256(wsf * 4);

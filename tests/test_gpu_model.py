@@ -394,3 +394,25 @@ def test_gate_up_rows_too_long_to_stream(tmp_path):
         assert max_rel(g.hidden(), o.hidden()) < 1e-4, pos
         assert_logits_parity(g.logits(), o.logits(), f"step {pos}")
     g.close()
+
+
+# The GEMM plan is a function of the prompt's own shape: a prompt gives the same
+# bits on a fresh model and after longer ones have grown the buffers (194 and 850
+# rows split differently when the buffer of another row count caps them; hidden 520
+# takes the single-stage kernel's splits)
+@pytest.mark.parametrize("hidden,inter,n,longer", [(512, 4352, 194, 275), (512, 4352, 850, 1024),
+                                                   (520, 4360, 130, 700)])
+def test_prefill_bits_do_not_depend_on_earlier_prompts(tmp_path, hidden, inter, n, longer):
+    s = shape_dict(hidden, 4, 1, 128, inter, 512, 1, 1e-6)
+    path = str(tmp_path / "m.safetensors")
+    write_safetensors(path, random_map(s, seed=n, std=0.05))
+    rng = np.random.default_rng(n)
+    ids, other = rng.integers(0, 512, n), rng.integers(0, 512, longer)
+    with myos.Model.open(path, to_block_shape(s), myos.KV_F32, longer) as m:
+        m.prefill(ids)
+        first = (m.logits(), m.hidden())
+        m.cache_clear()
+        m.prefill(other)
+        m.cache_clear()
+        m.prefill(ids)
+        assert np.array_equal(m.logits(), first[0]) and np.array_equal(m.hidden(), first[1])
