@@ -148,10 +148,11 @@ size_t gemm_ws_bound(int M, int N, int K);
 size_t gemm_ws_floats(int M, int N, int K);
 hipError_t launch_gemm(const GemmArgs &a, GemvEpi epi, hipStream_t s);
 // the op tier's Y[M, N] = X W^T with the NaN outputs recomputed as the
-// reference's chain; hi / lo are used where gemm_needs_planes says so
-bool gemm_needs_planes(const float *x, const uint16_t *w, int M, int N, int K);
+// reference's chain; hi / lo (lo right behind hi) are used where
+// gemm_needs_planes says so, ws holds gemm_ws_floats floats
+bool gemm_needs_planes(float *y, const uint16_t *w, const float *x, int M, int N, int K);
 hipError_t launch_gemm_op(float *y, const uint16_t *w, const float *x, int M, int N, int K, uint16_t *hi,
-                          uint16_t *lo, float *ws, size_t ws_cap, hipStream_t s);
+                          uint16_t *lo, float *ws, hipStream_t s);
 // EPI_RESID GEMM (y += A W^T) followed by the RMSNorm of y with gains g into
 // bf16 hi/lo planes, the split-K reduction and the norm in one pass when the
 // shape allows (else launch_gemm + launch_rmsnorm_rows_split)

@@ -3513,7 +3513,8 @@ GemmPlan gemm_plan(int M, int N, int K, size_t ws_cap) {
   return best;
 }
 
-// gemm_dma_kernel takes the call: 16-byte aligned operands, 32-bit row offsets,
+// gemm_dma_kernel takes the call: 16-byte aligned operands (launch_gemm_op sees to
+// a.x), 32-bit row offsets,
 // and for the epilogues on four columns at a time N and the head dim (so a
 // group stays in one head's q, k or v) multiples of 4 and aligned outputs
 template <int EPI>
@@ -3523,7 +3524,7 @@ static bool dm_ok(const GemmArgs &a) {
       if ((uintptr_t)p & (n - 1)) return false;
     return true;
   };
-  if (!aligned(16, {a.x, a.a_hi, a.a_lo, a.w}) || (size_t)a.M * a.K * 2 >= (1ull << 31) ||
+  if (!aligned(16, {a.a_hi, a.a_lo, a.w}) || (size_t)a.M * a.K * 2 >= (1ull << 31) ||
       (size_t)a.N * a.K * 2 >= (1ull << 31))
     return false;
   if (EPI == EPI_STORE) return true;
@@ -3699,38 +3700,57 @@ static hipError_t gemm_main(GemmArgs &a, hipStream_t s, int *splits_out) {
   return hipGetLastError();
 }
 
-// gemm_bf16's product. hi / lo: planes of M x K for the calls that need X split
-// (gemm_needs_planes); ws: gemm_ws_floats floats of partials.
-static bool gemm_op_direct(const GemmArgs &a) { return (a.K & 63) == 0 && dm_ok<EPI_STORE>(a); }
-bool gemm_needs_planes(const float *x, const uint16_t *w, int M, int N, int K) {
+// gemm_bf16's product. Its scratch (hi and lo, M x K bf16 each, lo right behind hi)
+// holds the planes of X, or on the tiles that split X themselves a copy of an X that
+// they cannot read in place: one off the 16-byte grid of their loads, or one that Y
+// overlaps, which other workgroups' outputs would overwrite. ws: gemm_ws_floats
+// floats of partials.
+static bool gemm_op_dma(const GemmArgs &a) { return (a.K & 63) == 0 && dm_ok<EPI_STORE>(a); }
+static bool gemm_op_xf(const GemmArgs &a) {
+  return gemm_op_dma(a) && kDm[gemm_plan(a.M, a.N, a.K, a.ws_cap).cfg].xf;
+}
+static bool gemm_op_copy(const GemmArgs &a) {
+  const uintptr_t x = (uintptr_t)a.x, y = (uintptr_t)a.y;
+  return (x & 15) || (x < y + (size_t)a.M * a.N * 4 && y < x + (size_t)a.M * a.K * 4);
+}
+static GemmArgs gemm_op_args(float *y, const uint16_t *w, const float *x, int M, int N, int K) {
   GemmArgs a{};
   a.x = x;
   a.w = w;
   a.M = M;
   a.N = N;
   a.K = K;
-  return !gemm_op_direct(a) || !kDm[gemm_plan(M, N, K, gemm_ws_floats(M, N, K)).cfg].xf;
+  a.y = y;
+  a.ws_cap = gemm_ws_floats(M, N, K);
+  return a;
+}
+bool gemm_needs_planes(float *y, const uint16_t *w, const float *x, int M, int N, int K) {
+  const GemmArgs a = gemm_op_args(y, w, x, M, N, K);
+  return !gemm_op_xf(a) || gemm_op_copy(a);
+}
+__global__ void __launch_bounds__(kBlock) copy_f32_kernel(float *dst, const float *src, size_t n) {
+  const size_t i = blockIdx.x * (size_t)kBlock + threadIdx.x;
+  if (i < n) dst[i] = src[i];
 }
 hipError_t launch_gemm_op(float *y, const uint16_t *w, const float *x, int M, int N, int K, uint16_t *hi,
-                          uint16_t *lo, float *ws, size_t ws_cap, hipStream_t s) {
-  GemmArgs g{};
-  g.x = x;
-  g.w = w;
-  g.M = M;
-  g.N = N;
-  g.K = K;
-  g.y = y;
+                          uint16_t *lo, float *ws, hipStream_t s) {
+  GemmArgs g = gemm_op_args(y, w, x, M, N, K);
   g.ws = ws;
-  g.ws_cap = ws_cap;
-  if (gemm_needs_planes(x, w, M, N, K)) {
+  const size_t n = (size_t)M * K;
+  hipError_t e = hipSuccess;
+  if (!gemm_op_xf(g)) {
     g.a_hi = hi;
     g.a_lo = lo;
-    hipError_t e = launch_split_rows(x, (size_t)M * K, hi, lo, s);
-    if (e != hipSuccess) return e;
+    e = launch_split_rows(x, n, hi, lo, s);
+  } else if (gemm_op_copy(g)) {
+    g.x = (float *)hi;
+    hipLaunchKernelGGL(copy_f32_kernel, dim3(nblk(n, kBlock)), dim3(kBlock), 0, s, (float *)hi, x, n);
+    e = hipGetLastError();
   }
-  hipError_t e = launch_gemm(g, EPI_STORE, s);
+  if (e != hipSuccess) return e;
+  e = launch_gemm(g, EPI_STORE, s);
   // gemm_dma_kernel and the reduction of its splits look for NaN themselves
-  return e == hipSuccess && !gemm_op_direct(g) ? launch_gemm_nan_repair(y, w, x, M, N, K, s) : e;
+  return e == hipSuccess && !gemm_op_dma(g) ? launch_gemm_nan_repair(y, w, x, M, N, K, s) : e;
 }
 
 hipError_t launch_gemm_resid_norm(const GemmArgs &args, const uint16_t *g, float eps,

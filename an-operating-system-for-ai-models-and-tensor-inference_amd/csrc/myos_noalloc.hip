@@ -90,7 +90,7 @@ int myos_gemm_bf16_noalloc(float *y, size_t y_len, const uint16_t *w, size_t w_l
   uint16_t *lo = (uint16_t *)(base + align256(x_need * 2));
   const size_t wsf = gemm_ws_floats((int)batch, (int)m, (int)k);
   float *ws = wsf ? (float *)(base + 2 * align256(x_need * 2)) : nullptr;
-  hipError_t e = launch_gemm_op(y, w, x, (int)batch, (int)m, (int)k, hi, lo, ws, wsf, s);
+  hipError_t e = launch_gemm_op(y, w, x, (int)batch, (int)m, (int)k, hi, lo, ws, s);
   return e == hipSuccess ? MYOS_OK : MYOS_E_HIP;
 }
 

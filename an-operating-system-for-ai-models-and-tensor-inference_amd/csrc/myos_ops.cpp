@@ -86,17 +86,17 @@ int myos_gemm_bf16(float *y, size_t y_len, const uint16_t *w, size_t w_len, cons
   if (k == 0) return hip_status(launch_fill_zero(y, y_need, S(stream)));
   if (batch > INT32_MAX || m > INT32_MAX || k > INT32_MAX) return MYOS_E_SHAPE;
   hipStream_t s = S(stream);
-  // the bf16 hi / lo planes of X, where the kernel does not split it itself, and
+  // the bf16 hi / lo planes of X, where the kernel does not read it in place, and
   // the partials of the K splits (none when the grid already fills the device)
   auto align256 = [](size_t n) { return (n + 255) & ~(size_t)255; };
   if (x_need > SIZE_MAX / 8) return MYOS_E_HIP;
-  const size_t plane = gemm_needs_planes(x, w, (int)batch, (int)m, (int)k) ? align256(x_need * 2) : 0;
+  const size_t plane = gemm_needs_planes(y, w, x, (int)batch, (int)m, (int)k) ? align256(x_need * 2) : 0;
   const size_t wsf = gemm_ws_floats((int)batch, (int)m, (int)k);
   OpScratch scr(2 * plane + wsf * 4, s);
   if (!scr.ok()) return MYOS_E_HIP;
   uint16_t *hi = (uint16_t *)scr.get(), *lo = hi + plane / 2;
   float *ws = wsf ? (float *)((uint8_t *)scr.get() + 2 * plane) : nullptr;
-  hipError_t e = launch_gemm_op(y, w, x, (int)batch, (int)m, (int)k, hi, lo, ws, wsf, s);
+  hipError_t e = launch_gemm_op(y, w, x, (int)batch, (int)m, (int)k, hi, lo, ws, s);
   const hipError_t f = scr.done();
   return hip_status(e != hipSuccess ? e : f);
 }

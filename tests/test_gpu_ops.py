@@ -409,3 +409,28 @@ def test_gemm_tiles(batch, m, k):
     # MFMA accumulation may not round to nearest: 4 gamma_k
     bound = (2.0 ** -17 + 4 * k * 2.0 ** -24) * mag
     assert bool(((y.double() - ref).abs() <= bound).all())
+
+
+# X off the 16-byte grid, and Y over X: the bits of the same call on aligned operands
+# of their own, through both entry points, on a tile that splits X itself whole and
+# in K splits, on one that reads planes of it, and on the single-stage kernel
+@pytest.mark.parametrize("call", [myos.gemm_bf16, myos.gemm_bf16_noalloc])
+@pytest.mark.parametrize("batch,m,k", [(37, 1536, 1536), (16, 256, 1536), (600, 4096, 512), (9, 70, 70)])
+def test_gemm_x_in_any_place(batch, m, k, call):
+    g = torch.Generator(device=DEV).manual_seed(batch + m)
+    w = (torch.randn(m, k, generator=g, device=DEV) * 0.02).to(torch.bfloat16)
+    x = torch.randn(batch, k, generator=g, device=DEV)
+    want = torch.full((batch, m), float("nan"), device=DEV)
+    call(want, w, x, batch, m, k)
+    for shift in (1, 2, 3):
+        xs = torch.empty(batch * k + shift, device=DEV)[shift:]
+        xs.copy_(x.flatten())
+        y = torch.full((batch, m), float("nan"), device=DEV)
+        call(y, w, xs, batch, m, k)
+        assert torch.equal(y, want), shift
+    # Y starts one row into X, and at X
+    for first in (0, k):
+        room = torch.zeros(batch * max(m, k) + k, device=DEV)
+        room[:batch * k] = x.flatten()
+        call(room[first:first + batch * m], w, room[:batch * k], batch, m, k)
+        assert torch.equal(room[first:first + batch * m].view(batch, m), want), first
