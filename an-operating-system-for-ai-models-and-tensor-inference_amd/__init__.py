@@ -82,6 +82,7 @@ EXPORTS = {
     "myos_attn_scale_f32": ([SZ, C.POINTER(F32)], I32),
     "myos_greedy_token": ([P, P, SZ, P], I32),
     "myos_stream_sync": ([P], I32),
+    "myos_scratch_trim": ([], None),
     "myos_block_shape_preset": ([I32, C.POINTER(BlockShape)], I32),
     "myos_model_open": ([C.c_char_p, C.POINTER(BlockShape), I32, SZ, C.POINTER(P)], I32),
     "myos_model_close": ([P], None),
@@ -344,6 +345,11 @@ def greedy_token(logits, out=None, stream=None) -> int:
     _check(lib().myos_greedy_token(op, lp, ln, s), "greedy_token")
     _check(lib().myos_stream_sync(s), "greedy_token sync")
     return int(out.view(torch.int32).cpu()[0].item()) & 0xFFFFFFFF
+
+
+def scratch_trim():
+    """Give the op calls' idle scratch on the current device back."""
+    lib().myos_scratch_trim()
 
 
 # ------------------------------------------------------------- model tier ----

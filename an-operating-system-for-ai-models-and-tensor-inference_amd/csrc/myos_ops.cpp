@@ -53,6 +53,8 @@ int myos_stream_sync(myos_stream_t stream) {
   return hip_status(hipStreamSynchronize(S(stream)));
 }
 
+void myos_scratch_trim(void) { op_scratch_trim(); }
+
 // bf16.rs:94-122
 int myos_gemv_bf16(float *y, size_t y_len, const uint16_t *w, size_t w_len, const float *x,
                    size_t x_len, size_t m, size_t k, myos_stream_t stream) {

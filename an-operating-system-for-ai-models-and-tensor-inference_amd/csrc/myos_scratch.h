@@ -9,10 +9,12 @@
 // what makes reuse safe: a handle that a later stream reuses waits for the
 // earlier stream's work.
 //
-// Bounded: at most kScratchBlocks blocks and kScratchBytes per device. Beyond
-// that, under stream capture, and where a block cannot be had, a call takes
-// hipMallocAsync / hipFreeAsync. op_scratch_trim (a closing model calls it)
-// gives idle blocks back.
+// Bounded: at most kScratchBlocks blocks and kScratchBytes per device. At a bound, a
+// block that no call has taken for kScratchIdle calls (its stream is gone, or its
+// shapes are) makes room: it is freed in stream order behind its event. With none,
+// under stream capture, and where a block cannot be had, a call takes hipMallocAsync
+// / hipFreeAsync. op_scratch_trim (myos_scratch_trim, and a closing model) gives idle
+// blocks back.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -37,6 +39,7 @@ class OpScratch {
   void *block_ = nullptr;  // the kept block, null for a plain allocation
 };
 
+// frees the current device's blocks that no call holds, waiting for their last work
 void op_scratch_trim();
 
 }  // namespace myos

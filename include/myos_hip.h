@@ -173,6 +173,12 @@ int myos_greedy_token(uint32_t *out, const float *logits, size_t n, myos_stream_
 /* Block until the stream's work is done; returns MYOS_E_HIP on a device error. */
 int myos_stream_sync(myos_stream_t stream);
 
+/* Give the op tier's idle scratch on the current device back, waiting for its
+ * last calls' work. gemm_bf16, gqa_attn_f32 and greedy_token keep scratch between
+ * calls, a block per stream, at most 8 and 256 MiB per device; closing a model
+ * does this too. No counterpart in the reference. */
+void myos_scratch_trim(void);
+
 /* ======================= model tier (model_core) ===================== */
 
 typedef struct myos_model myos_model;

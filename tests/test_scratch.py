@@ -1,0 +1,138 @@
+"""The op tier's kept scratch blocks (csrc/myos_scratch.cpp) on the CPU, built against a
+stand-in for the HIP calls that counts allocations and can fail them."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "an-operating-system-for-ai-models-and-tensor-inference_amd", "csrc")
+
+HIP = r"""
+#pragma once
+#include <stdint.h>
+#include <stdlib.h>
+#include <set>
+typedef int hipError_t;
+typedef struct S *hipStream_t;
+typedef struct E { bool recorded; } *hipEvent_t;
+enum { hipSuccess = 0, hipErrorOutOfMemory = 2 };
+enum hipStreamCaptureStatus { hipStreamCaptureStatusNone };
+enum { hipEventDisableTiming = 2 };
+inline std::set<void *> live;
+inline int mallocs, last_error, fail_mallocs;
+inline void (*on_sync)() = nullptr;
+inline hipError_t hipGetDevice(int *d) { *d = 0; return 0; }
+inline hipError_t hipGetLastError() { int e = last_error; last_error = 0; return e; }
+inline hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c) { *c = hipStreamCaptureStatusNone; return 0; }
+inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t e, int) { return e->recorded ? 0 : (last_error = 1); }
+inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, int) { *e = new E{false}; return 0; }
+inline hipError_t hipEventDestroy(hipEvent_t e) { delete e; return 0; }
+inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { e->recorded = true; return 0; }
+inline hipError_t hipEventSynchronize(hipEvent_t) { if (on_sync) on_sync(); return 0; }
+inline hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) {
+  if (fail_mallocs > 0) { fail_mallocs--; return last_error = hipErrorOutOfMemory; }
+  mallocs++;
+  live.insert(*p = malloc(1));
+  return 0;
+}
+inline hipError_t hipFree(void *p) { if (!live.erase(p)) abort(); free(p); return 0; }
+inline hipError_t hipFreeAsync(void *p, hipStream_t) { return hipFree(p); }
+"""
+
+MAIN = r"""
+#include "myos_scratch.h"
+#include <chrono>
+#include <future>
+#include <stdio.h>
+#include <string.h>
+using myos::OpScratch;
+#define CHECK(c) do { if (!(c)) { printf("line %d: %s\n", __LINE__, #c); exit(1); } } while (0)
+static hipStream_t stream(long i) { return (hipStream_t)(i * 64); }
+static void call(long s, size_t bytes = 1000) {
+  OpScratch x(bytes, stream(s));
+  CHECK(x.ok() && x.get());
+  CHECK(x.done() == hipSuccess);
+}
+// calls of stream s that allocate, of ten
+static int allocs(long s, size_t bytes = 1000) {
+  const int before = mallocs;
+  for (int i = 0; i < 10; i++) call(s, bytes);
+  return mallocs - before;
+}
+int main(int, char **argv) {
+  const char *what = argv[1];
+  if (!strcmp(what, "dead_streams")) {
+    // blocks of streams that never call again make room for a later stream's, in
+    // number and in size; streams taking turns never lose theirs
+    for (long s = 1; s <= 8; s++) call(s);
+    CHECK(allocs(9) == 10);
+    for (int i = 0; i < 300; i++) call(1);
+    CHECK(allocs(9) <= 1);
+    CHECK(allocs(1) == 0);
+    for (long s = 20; s < 26; s++) allocs(s);
+    call(30, 200u << 20);
+    for (int i = 0; i < 300; i++) call(1);
+    CHECK(allocs(31, 200u << 20) <= 1);
+    CHECK(allocs(1) == 0);
+    const int before = mallocs;
+    for (int i = 0; i < 1000; i++)
+      for (long s = 40; s < 52; s++) call(s);
+    CHECK(live.size() <= 8 && mallocs - before < 12 * 1000 && allocs(31, 200u << 20) <= 10);
+  } else if (!strcmp(what, "failed_block")) {
+    // the kept block cannot be had, the plain allocation can: the call goes on, with
+    // no error left for the launches after it to find
+    fail_mallocs = 1;
+    OpScratch x(1000, stream(1));
+    CHECK(x.ok() && x.get());
+    CHECK(hipGetLastError() == hipSuccess);
+    CHECK(x.done() == hipSuccess && live.empty());
+  } else if (!strcmp(what, "trim")) {
+    // idle blocks are given back, held ones stay, and other calls go on during the
+    // wait for a block's work
+    call(1);
+    call(2, 64u << 20);
+    OpScratch held(1000, stream(3));
+    on_sync = [] {
+      auto f = std::async(std::launch::async, [] { call(4); });
+      if (f.wait_for(std::chrono::seconds(5)) != std::future_status::ready) {
+        printf("a call waits for the trim\n");
+        fflush(stdout);
+        _exit(1);
+      }
+    };
+    myos::op_scratch_trim();
+    on_sync = nullptr;
+    myos::op_scratch_trim();
+    CHECK(live.size() == 1);
+    CHECK(held.done() == hipSuccess);
+    myos::op_scratch_trim();
+    CHECK(live.empty());
+    call(1);
+    CHECK(live.size() == 1);
+  } else {
+    return 2;
+  }
+  return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    d = tmp_path_factory.mktemp("scratch")
+    (d / "hip").mkdir()
+    (d / "hip" / "hip_runtime.h").write_text(HIP)
+    (d / "main.cpp").write_text("#include <unistd.h>\n" + MAIN)
+    out = str(d / "t")
+    subprocess.run(["g++", "-std=c++17", "-g", "-fsanitize=address,undefined", "-I", str(d), "-I", CSRC,
+                    str(d / "main.cpp"), os.path.join(CSRC, "myos_scratch.cpp"), "-o", out, "-lpthread"],
+                   check=True)
+    return out
+
+
+@pytest.mark.parametrize("case", ["dead_streams", "failed_block", "trim"])
+def test_scratch(exe, case):
+    r = subprocess.run([exe, case], capture_output=True, text=True, timeout=60,
+                       env={**os.environ, "ASAN_OPTIONS": "detect_leaks=0"})
+    assert r.returncode == 0, r.stdout + r.stderr
