@@ -1678,10 +1678,10 @@ __device__ __forceinline__ int dm_swz(int r) {
 // 64 lanes x 16 bytes from base + voff (per lane) into LDS at lds, lds + 16, ...
 // No destination register: completion is counted by vmcnt and waited for in
 // dm_wait. (The builtin would make the compiler drain every load before the
-// next LDS read.)
+// next LDS read.) m0, the LDS address, is an input, so the compiler knows of the
+// write; one wait state lies between the two.
 __device__ __forceinline__ void dm_load(uint32_t lds, uint32_t voff, const void *base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base)
-               : "memory");
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(voff), "s"(base) : "memory");
 }
 // this wave's loads but the last N have landed and its LDS reads are done;
 // after the barrier that holds for every wave
