@@ -1821,10 +1821,11 @@ __global__ void __launch_bounds__(kBlock) split8_kernel(const float *X, size_t n
 // right from +0, each product rounded before it is added) gives +-inf; so an
 // output that is NaN is recomputed as that chain.
 __device__ float gemm_chain(const float *x, const uint16_t *w, int row, int col, int K) {
+#pragma clang fp contract(off)  // __fadd_rn of __fmul_rn alone becomes one fma
   const uint16_t *wr = w + (size_t)col * K;
   const float *xr = x + (size_t)row * K;
   float acc = 0.f;
-  for (int j = 0; j < K; j++) acc = __fadd_rn(acc, __fmul_rn(bf16f(wr[j]), xr[j]));
+  for (int j = 0; j < K; j++) acc += bf16f(wr[j]) * xr[j];
   return acc;
 }
 

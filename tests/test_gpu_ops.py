@@ -434,3 +434,40 @@ def test_gemm_x_in_any_place(batch, m, k, call):
         room[:batch * k] = x.flatten()
         call(room[first:first + batch * m], w, room[:batch * k], batch, m, k)
         assert torch.equal(room[first:first + batch * m].view(batch, m), want), first
+
+
+# The outputs that meet an infinity, a NaN or an activation beyond bf16's range, in the
+# first and last rows and columns, against the reference's chain: by the tile kernel's
+# two epilogues (16 x 64, 128 x 128; 128 x 384, 256 x 256), by both reductions of K
+# splits (N % 4 == 0 and not; 32 x 64 and 256 x 256), and by the pass after the
+# single-stage kernel
+@pytest.mark.parametrize("batch,m,k", [(442, 458, 1664), (566, 5227, 64), (1207, 7514, 128), (1035, 11363, 64),
+                                       (33, 164, 3712), (33, 169, 3712), (2047, 3584, 4096), (390, 8565, 4224),
+                                       (130, 71, 100)])
+def test_gemm_non_finite(batch, m, k):
+    rng = np.random.default_rng(batch + m + k)
+    w = rand_w(rng, m, k)
+    x = rng.standard_normal((batch, k), dtype=np.float32)
+    clean_w, clean_x = dev(w, torch.int16).view(torch.bfloat16), dev(x)
+    w[m - 1, 0], w[m // 2, k - 1], w[0, 5] = 0x7F80, 0x7FC0, 0xFF80  # inf, NaN, -inf
+    x[::2, 0] = 2.0  # no lo part: the infinite weight meets a zero there
+    x[1, 5] = 0.0    # inf times zero: the chain's NaN
+    x[batch - 1, 3], x[0, k - 1] = np.inf, 3.4e38
+    y = torch.full((batch, m), 7.0, device=DEV)
+    myos.gemm_bf16(y, dev(w, torch.int16), dev(x), batch, m, k)
+    got = host(y)
+    rows, cols = [0, batch - 1], [0, m // 2, m - 1]
+    with np.errstate(all="ignore"):
+        want_r = oracle.gemm_bf16(w, x[rows], 2, m, k, threads=8)
+        want_c = oracle.gemm_bf16(w[cols], x, batch, 3, k, threads=8)
+    assert np.array_equal(got[rows], want_r, equal_nan=True)
+    assert np.array_equal(got[:, cols], want_c, equal_nan=True)
+    assert np.isinf(want_c[:, 2]).sum() > batch // 3 and np.isfinite(want_r[0]).sum() > m - 4
+    # the others: the finite product, with x[:, 0] as the call had it
+    clean_x[::2, 0], clean_x[1, 5] = 2.0, 0.0
+    ref = torch.mm(clean_x.double(), clean_w.double().t().contiguous())
+    mag = torch.mm(clean_x.double().abs(), clean_w.double().abs().t().contiguous())
+    bound = (2.0 ** -17 + 4 * k * 2.0 ** -24) * mag
+    ok = ((y.double() - ref).abs() <= bound).cpu().numpy()
+    ok[rows], ok[:, cols] = True, True
+    assert ok.all()
