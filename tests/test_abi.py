@@ -272,3 +272,18 @@ def test_prefill_plan_fits_the_bound(L):
             need = max(need, splits * m * n if splits > 1 else 0)
             if m % 37 == 1 or m in (128, 1024, 2048):
                 assert need <= bound(m, n, k), (m, n, k)
+
+
+def test_gemm_tile_shapes_reach_every_tile(L):
+    # the shapes of the GPU test of gemm_bf16's tiles, by the op's own plan: every tile
+    # whole and split, but for one that the plan never splits
+    from test_gpu_ops import TILE_SHAPES
+    plan, ws = L._ZN4myos9gemm_planEiiim, L._ZN4myos14gemm_ws_floatsEiii
+    plan.argtypes, plan.restype = [C.c_int] * 3 + [C.c_size_t], C.c_uint64
+    ws.argtypes, ws.restype = [C.c_int] * 3, C.c_size_t
+    seen = set()
+    for shape in TILE_SHAPES:
+        p = plan(*shape, ws(*shape))
+        seen.add((p & 0xFFFFFFFF, p >> 32 > 1))
+    tiles, wide160 = 15, 5
+    assert {(c, s) for c in range(tiles) for s in (False, True)} - seen <= {(wide160, True)}

@@ -385,18 +385,23 @@ def test_scratch_streams_and_threads():
     assert not bad
 
 
-# gemm_bf16 over the direct-to-LDS tiles: each tile of the plan whole and (where
-# the plan splits it) in K splits, with row and column remainders: 64 x 80,
-# 16 x 64, 16 x 80, 32 x 64, 32 x 80, 64 x 64, 64 x 128, 128 x 64, 128 x 80,
-# 128 x 96, 128 x 128, 128 x 160, 128 x 384, 128 x 512, 256 x 256; N % 4 != 0
-# (scalar stores), one row, one K step, 8 or more M tiles (XCD runs)
-@pytest.mark.parametrize("batch,m,k", [
+# gemm_bf16 over the direct-to-LDS tiles: each tile whole and, but for 128 x 160, which
+# the plan never splits, in K splits (test_abi.py checks that against the plan), with
+# row and column remainders, N % 4 != 0 (scalar stores), one row, one K step, 8 or more
+# M tiles (XCD runs)
+TILE_SHAPES = [
     (2, 3515, 320), (34, 386, 1600), (66, 4269, 2112), (442, 458, 1664), (3, 671, 1536),
     (244, 637, 2304), (39, 6293, 2368), (985, 350, 128), (90, 1510, 1856), (205, 1465, 768),
     (140, 3545, 1536), (1012, 979, 384), (1, 3203, 2176), (757, 6394, 192), (21, 1535, 2176),
     (305, 67, 2176), (527, 3087, 256), (513, 1240, 1600), (596, 3666, 512), (78, 2018, 2240),
     (566, 5227, 64), (1207, 7514, 128), (2047, 8203, 448), (381, 37888, 192), (128, 20479, 320),
-    (2048, 1536, 8960), (1, 1, 64)])
+    (2048, 1536, 8960), (1, 1, 64),
+    (130, 81, 1920), (195, 82, 2432), (266, 82, 3264), (131, 1383, 1984), (33, 453, 2688),
+    (130, 10333, 64), (1035, 11363, 64), (390, 8565, 4224), (2047, 3584, 4096), (1, 9615, 4160),
+    (1, 4909, 4672)]
+
+
+@pytest.mark.parametrize("batch,m,k", TILE_SHAPES)
 def test_gemm_tiles(batch, m, k):
     g = torch.Generator(device=DEV).manual_seed(batch + m + k)
     w = (torch.randn(m, k, generator=g, device=DEV) * 0.02).to(torch.bfloat16)
