@@ -725,8 +725,9 @@ __global__ void __launch_bounds__(kBlock) attn_decode_d128_kernel(AttnDecodeArgs
   if (attn_last_in_group(a, g, nv)) attn_merge(a, g, gq, D, nv, nchunks, smem);
 }
 
-// Decode attention at head_dim 128 over a cache of at most 256 positions: one
-// workgroup per query head, no chunks to merge. 16-lane group r0 of 32 holds rows
+// Decode attention at head_dim 128 for a cache of at most 256 positions (its
+// capacity: the launch is recorded once and does not know the position; a larger
+// cache keeps the chunk kernel at every position): one workgroup per query head, no chunks to merge. 16-lane group r0 of 32 holds rows
 // r0 + 32 u of K and of V, columns 4 l .. + 3 and 64 + 4 l .. + 3 each, so every
 // load goes out at once, before the position is known; every wave takes the
 // softmax of the whole row, and the 32 groups' V sums are added through LDS. The
@@ -3311,9 +3312,11 @@ hipError_t launch_rope_apply_tab(float *x, size_t len, size_t head_dim, const Ro
 
 // Positions per chunk of gqa_chunk_kernel: one chunk per head, with no scratch and
 // no merge launch, while a head's K and V are at most 1 MB and its scores fit LDS
-// (12 q / 2 kv heads of 128: 300 positions 11.9 -> 6.6 us a call, 1024 positions
-// 14.2 -> 11.6 among others and 25.5 -> 25.3 waited for alone); beyond, about two
-// chunks per CU over all heads, 32 to kGqaMaxChunk positions each.
+// (12 q / 2 kv heads of 128, K and V in the caches as a repeated call leaves them:
+// 300 positions 11.9 -> 6.6 us a call, 1024 positions 14.2 -> 11.6 among others and
+// 25.5 -> 25.3 waited for alone; not measured with K and V in HBM, where one CU
+// streams 28-30 GB/s, nor at other head counts); beyond, about two chunks per CU
+// over all heads, 32 to kGqaMaxChunk positions each.
 static int gqa_chunk(int nq, int d, int seen) {
   if (seen <= kGqaMaxChunk && seen * d <= 128 * kGqaMaxChunk) return kGqaMaxChunk;
   const long per = (512 + nq - 1) / nq;  // chunks per head
@@ -3433,9 +3436,10 @@ constexpr int kCUs = 256;
 // gemm_dma_kernel's tiles, with the microseconds a 64-wide K step takes on one
 // CU (fitted to kernel times of this tile on MI355X over 8 to 8192 rows of the
 // 1.5B and 7B projections and of larger products). Eight waves with
-// alternating groups for the wide tiles; for few rows, tiles no taller than
-// the rows, whose time is the latency of their loads (there the alternation
-// measured slower: 7B gate/up at 128 rows on 128 x 160, 83 us against 91).
+// alternating groups for the wide tiles and the eight-wave 64-row ones; for few
+// rows, tiles no taller than the rows, whose time is the latency of their loads (on
+// the other narrow tiles the alternation measured slower: 7B gate/up at 128 rows on
+// 128 x 160, 83 us against 91).
 using Dm256x256 = DmCfg<4, 8, 4, 2, 1, 32, 3, true>;
 using Dm128x512 = DmCfg<4, 8, 2, 4, 1, 32, 3, true>;
 using Dm128x384 = DmCfg<4, 6, 2, 4, 1, 32, 4, true>;
@@ -3933,7 +3937,7 @@ const char *kernel_build_info() {
   return "gfx950; gemv: wave/workgroup teams, 16B nontemporal bf16 loads, fused "
          "rmsnorm/bias+rope+kv/swiglu/residual/argmax epilogues; attention: split-position "
          "decode partials merged by the last chunk workgroup of each kv group; streaming GEMV for "
-         "large projections; prefill: v_mfma_f32_32x32x16_bf16 hi/lo GEMM, LDS-pipelined, planned tiles";
+         "large projections; prefill: v_mfma_f32_16x16x32_bf16 hi/lo GEMM, direct-to-LDS loads, planned tiles";
 }
 
 }  // namespace myos

@@ -1,9 +1,9 @@
 // gemm_bf16 without any allocation: myos_gemm_bf16_noalloc.
 //
-// myos_gemm_bf16 allocates its scratch on every call (the bf16 hi / lo planes
-// of X and the f32 partials of the K splits, hipMallocAsync / hipFreeAsync).
-// Callers that cannot allocate -- code under stream capture, tight serving
-// loops -- use this variant instead: the same kernels, with the scratch in a
+// myos_gemm_bf16 keeps scratch per stream between calls, and allocates it on a
+// stream's first call, when it must grow and under stream capture (the bf16 hi /
+// lo planes of X and the f32 partials of the K splits). Callers that cannot
+// allocate use this variant instead: the same kernels, with the scratch in a
 // file-scope device array of kScratchBytes per GPU, held until the process
 // ends. Host code never passes the array's name to a kernel (on the host it
 // is only a stand-in symbol): each device's address of it is looked up once
@@ -11,8 +11,8 @@
 //
 // Every call on one GPU shares that GPU's array; calls that overlap on one
 // GPU (two streams, two threads) race on it. Nothing in it has to start at
-// zero: each call writes every scratch word it reads (the split kernel both
-// planes, each K split its own partial tile) before reading it.
+// zero: each call writes every scratch word it reads (both planes, or a copy of
+// X; each K split its own partial tile) before reading it.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
