@@ -138,11 +138,10 @@ struct GemmPlan {
   int splits = 1;
 };
 GemmPlan gemm_plan(int M, int N, int K, size_t ws_cap);
-// partial-buffer floats that no plan for up to M rows exceeds: the model's products
-// are planned by their shape alone, and the need does not grow with the rows, so a
-// buffer sized by the longest prompt's own plan would not hold (or, capping the
-// plan, would change the sums of) a shorter one
-size_t gemm_ws_bound(int M, int N, int K);
+// partial-buffer floats of the model's product of this shape (0: one split). It is
+// planned by its shape alone, so its sums do not depend on the calls before it; the
+// need does not grow with the rows: the buffer of a longer prompt may be too small
+size_t gemm_ws_need(int M, int N, int K);
 // the partial-buffer floats of the op tier's product (0: one split); a function of
 // the shape as well
 size_t gemm_ws_floats(int M, int N, int K);

@@ -1668,7 +1668,7 @@ struct DmCfg {
   static constexpr int EPL = WK > 1 ? WK * TILE : 0;  // partial tiles at the end
   static constexpr int LDS = NST * STAGE > EPL ? NST * STAGE : EPL;
   static constexpr int KP = KS / 32 / WK;          // 32-wide K parts per wave and stage
-  static_assert(BM * BN <= 256 * 256 && BM % RPI == 0 && BN % RPI == 0 && LDS <= 160 * 1024 && KP >= 1 && NST >= 2, "tile");
+  static_assert(BM % RPI == 0 && BN % RPI == 0 && LDS <= 160 * 1024 && KP >= 1 && NST >= 2, "tile");
   static_assert(LPW * (NST - 2) < 63, "vmcnt");
 };
 template <int CPR>
@@ -3609,35 +3609,9 @@ static int gemm_scratch_splits(int M, int N, int K) {
   return best;
 }
 
-// Up to 256 rows the plans are gone through (30 us of host time for four 1.5B
-// projections; the bound of any shape would take 64 MB): within sixteen rows every
-// tile keeps its count and a plan's time only grows with the rows, so a plan that is
-// slower at the first of them than another at the last is never the cheapest. Beyond,
-// where the sum over the splits comes near it anyway (2048 rows: 370 us for the last
-// percent), that bound: sp splits of T tiles fill at most one round, sp M N <= sp T bm
-// bn <= kCUs bm bn, and the single-stage kernel's sp <= 512 / T + 1 with sp > 1 stays
-// below 1024 of its tiles; neither splits beyond the 64-wide steps.
-size_t gemm_ws_bound(int M, int N, int K) {
-  constexpr size_t kAny = (size_t)kCUs * 256 * 256;
-  static_assert(1024 * GBM * GBN <= kAny, "the single-stage kernel's splits");
-  const size_t steps = ((size_t)K + 63) / 64;
-  if (steps <= 1) return 0;
-  if (M > 256) return std::min(kAny, steps * M * N);
-  size_t need = 0;
-  for (long m = 1; m <= M; m++) {
-    const int sp = gemm_splits_old((int)m, N, K);
-    if (sp > 1) need = std::max(need, (size_t)sp * m * N);
-  }
-  if (K & 63) return need;
-  for (long lo = 1; lo <= M; lo += 16) {
-    const int hi = (int)std::min<long>(lo + 15, M);
-    double best = 1e30;
-    each_plan(hi, N, K, SIZE_MAX, [&](int c, int sp) { best = std::min(best, dm_cost(c, hi, N, K, sp)); });
-    each_plan((int)lo, N, K, SIZE_MAX, [&](int c, int sp) {
-      if (sp > 1 && dm_cost(c, (int)lo, N, K, sp) <= best) need = std::max(need, (size_t)sp * hi * N);
-    });
-  }
-  return need;
+size_t gemm_ws_need(int M, int N, int K) {
+  const int sp = std::max(gemm_plan(M, N, K, SIZE_MAX).splits, gemm_splits_old(M, N, K));
+  return sp > 1 ? (size_t)sp * M * N : 0;
 }
 
 size_t gemm_ws_floats(int M, int N, int K) {
@@ -3700,7 +3674,7 @@ static hipError_t go_dm_cfg(const GemmArgs &a, int cfg, int splits, int ncols, h
 template <int EPI>
 static hipError_t gemm_main(GemmArgs &a, hipStream_t s, int *splits_out) {
   // the op tier's product plans within the scratch its entry points state; the
-  // model's by their shape alone, in a buffer of gemm_ws_bound floats
+  // model's by their shape alone, in a buffer of gemm_ws_need floats
   const size_t cap = EPI != EPI_STORE ? SIZE_MAX : a.ws ? a.ws_cap : 0;
   const GemmPlan p = dm_ok<EPI>(a) ? gemm_plan(a.M, a.N, a.K, cap) : GemmPlan();
   if (p.cfg >= 0) {

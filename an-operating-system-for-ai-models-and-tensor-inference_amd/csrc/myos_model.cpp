@@ -355,26 +355,34 @@ int write_state(myos_model *m, uint32_t pos, uint32_t token, uint32_t step, uint
   return MYOS_OK;
 }
 
+// floats of the partials' buffer for a prompt of `rows` ids: the K splits of the
+// four projections; the attention's key splits use the same space between them
+size_t prefill_ws_need(const myos_model *m, size_t rows) {
+  const size_t H = m->s.hidden, I = m->s.intermediate, Q = m->q_dim;
+  const size_t proj[4][2] = {{m->qkv_rows, H}, {H, Q}, {m->gu_rows, H}, {H, I}};
+  size_t need = 0;
+  for (auto &nk : proj) need = std::max(need, gemm_ws_need((int)rows, (int)nk[0], (int)nk[1]));
+  if (m->s.head_dim == 128) need = std::max(need, attn_prefill_part_floats((int)m->s.num_q_heads, (int)rows, 4));
+  return need;
+}
+
+// one block for both (two large ones are slower to allocate: a new model's first
+// 2048 ids 3.39 -> 3.70 ms)
 int ensure_prefill(myos_model *m, size_t rows) {
-  if (rows <= m->pf_rows) return MYOS_OK;
+  size_t wsf = prefill_ws_need(m, rows);
+  if (rows <= m->pf_rows && wsf <= m->pws_cap) return MYOS_OK;
+  rows = std::max(rows, m->pf_rows);
+  wsf = std::max(wsf, m->pws_cap);
   if (m->pf) {
     HIP_TRY(hipStreamSynchronize(m->stream));
+    m->pf_rows = m->pws_cap = 0;
     HIP_TRY(hipFree(m->pf));
     m->pf = nullptr;
-    m->pf_rows = 0;
   }
   const size_t H = m->s.hidden, I = m->s.intermediate, Q = m->q_dim;
   const size_t bx = align256(rows * H * 4), bq = align256(rows * Q * 4);
   const size_t ba = align256(rows * (H > Q ? H : Q) * 2), bh = align256(rows * I * 2);
-  const size_t bt = align256(rows * 4);
-  // K-split partials of the four projections, for any prompt of up to `rows` ids
-  const int R = (int)rows;
-  size_t wsf = 0;
-  const size_t proj[4][2] = {{m->qkv_rows, H}, {H, Q}, {m->gu_rows, H}, {H, I}};
-  for (auto &nk : proj) wsf = std::max(wsf, gemm_ws_bound(R, (int)nk[0], (int)nk[1]));
-  // the attention's key-split partials use the same space (between GEMMs)
-  if (m->s.head_dim == 128) wsf = std::max(wsf, attn_prefill_part_floats((int)m->s.num_q_heads, R, 4));
-  const size_t bw = align256(wsf * 4);
+  const size_t bt = align256(rows * 4), bw = align256(wsf * 4);
   const size_t total = bx + bq + 2 * ba + 2 * bh + bt + bw;
   HIP_TRY(hipMalloc((void **)&m->pf, total));
   uint8_t *p = m->pf;
